@@ -478,6 +478,18 @@ namespace mi
     {
       return;
     }
+    if (a.chunk_scratch != nullptr && chunk_applies(kv, a))
+    {
+      AttentionArgs full = a;
+      full.seq_k = std::max(a.seq_k, a.capacity);
+      void *scratch = a.chunk_scratch->take(stream, chunk_workspace_bytes(kv, a),
+                                            chunk_workspace_bytes(kv, full));
+      if (scratch != nullptr)
+      {
+        launch_chunk(kv, a, scratch, stream);
+        return;
+      }
+    }
     if (prefill_applies(kv, a))
     {
       launch_prefill(kv, a, stream);

@@ -305,6 +305,19 @@ namespace mi
   // share one; launches on one stream are ordered by it.
   float *stream_workspace(hipStream_t stream, std::size_t count);
 
+  // Scratch of a chunk's attention (chunk.hip): at least `bytes` that are the
+  // launches' on `stream` until the next request for that stream, or null
+  // where none can be had (the launch then takes the path that needs none).
+  // `growing_to`: the bytes the same queries would need once the owner is
+  // full, so that a prompt's chunks do not outgrow it one after the other.
+  struct StreamScratch
+  {
+    virtual void *take(hipStream_t stream, std::size_t bytes, std::size_t growing_to) = 0;
+
+  protected:
+    ~StreamScratch() = default;
+  };
+
   struct AttentionArgs
   {
     const std::uint16_t *q;   // (seq_q, heads, hd) fp16
@@ -327,6 +340,8 @@ namespace mi
     float *partials;          // attention_partials_floats(hd) or null: no split
     std::size_t partials_floats; // its size, when the caller knows it (0: unknown)
     WorkspaceSource *workspace;  // the decode path's scratch, or null (see above)
+    StreamScratch *chunk_scratch; // a chunk's laid-out pages go here, or null: none
+    int capacity;                // the positions the owner has room for; with chunk_scratch
   };
 
   // How a launch given partials splits its keys: runs and keys a run.
@@ -347,6 +362,16 @@ namespace mi
   // does not.
   bool prefill_applies(const KVSource &kv, const AttentionArgs &a);
   void launch_prefill(const KVSource &kv, const AttentionArgs &a, hipStream_t stream);
+
+  // The chunk path over laid-out pages (chunk.hip): what prefill_applies
+  // takes, of a paged or sealing cache and at least kChunkQueries queries.
+  // `workspace` holds chunk_workspace_bytes and belongs to the launch until
+  // the stream is past it.
+  constexpr int kChunkQueries = 64;
+  bool chunk_applies(const KVSource &kv, const AttentionArgs &a);
+  std::size_t chunk_workspace_bytes(const KVSource &kv, const AttentionArgs &a);
+  void launch_chunk(const KVSource &kv, const AttentionArgs &a, void *workspace,
+                    hipStream_t stream);
 
   // The decode fast path (decode.hip) over `layers` consecutive layers of one
   // cache in one launch. Layer first_layer + i reads its page addresses and

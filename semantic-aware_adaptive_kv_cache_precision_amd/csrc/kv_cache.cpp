@@ -1152,6 +1152,8 @@ namespace mi
     a.partials = partials;
     a.partials_floats = partials != nullptr ? attention_partials_floats(head_dim) : 0;
     a.workspace = &workspace_;
+    a.chunk_scratch = &chunk_scratch_;
+    a.capacity = capacity_tokens();
     KVSource kv{};
     kv.page_tokens = page_tokens_;
     const std::size_t row = static_cast<std::size_t>(layer) * table_.stride();

@@ -107,6 +107,47 @@ namespace mi
     }
   }
 
+  void *StreamBuffers::take(hipStream_t stream, std::size_t bytes, std::size_t growing_to)
+  {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capturing) != hipSuccess)
+    {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    if (capturing != hipStreamCaptureStatusNone)
+    {
+      return nullptr;
+    }
+    std::lock_guard<std::mutex> hold(lock_);
+    auto at = std::find_if(held_.begin(), held_.end(),
+                           [&](const auto &entry) { return entry.first == stream; });
+    if (at == held_.end())
+    {
+      if (held_.size() == kMost)
+      {
+        return nullptr;
+      }
+      held_.emplace_back(stream, nullptr);
+      at = held_.end() - 1;
+    }
+    std::unique_ptr<DeviceBuffer> &buffer = at->second;
+    if (buffer == nullptr || buffer->bytes() < bytes)
+    {
+      buffer.reset(); // waits for launches that use it
+      try
+      {
+        buffer = std::make_unique<DeviceBuffer>(std::max(bytes, growing_to));
+      }
+      catch (const OutOfMemory &)
+      {
+        (void)hipGetLastError();
+        return nullptr;
+      }
+    }
+    return buffer->raw();
+  }
+
   const void *UploadBuffer::send_bytes(const void *host, std::size_t bytes, hipStream_t stream)
   {
     if (bytes == 0)

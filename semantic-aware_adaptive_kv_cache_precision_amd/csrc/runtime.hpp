@@ -134,6 +134,24 @@ namespace mi
     std::vector<std::unique_ptr<DeviceBuffer>> outgrown_;
   };
 
+  // A buffer a stream, of one owner's, for launches that hand data to each
+  // other on that stream alone. Bounded: kMost streams (a buffer each, as
+  // large as its largest request); a further stream gets none, nor does a
+  // stream that is being captured, whose graph could be replayed beside
+  // other work of the owner's, nor a request the device has no memory for.
+  // Grown buffers and the owner's end give the old ones back, once the
+  // device is idle. Safe with several threads.
+  class StreamBuffers final : public StreamScratch
+  {
+  public:
+    void *take(hipStream_t stream, std::size_t bytes, std::size_t growing_to) override;
+
+  private:
+    static constexpr std::size_t kMost = 4;
+    std::mutex lock_;
+    std::vector<std::pair<hipStream_t, std::unique_ptr<DeviceBuffer>>> held_;
+  };
+
   // Test hook: the next `n` granule maps fail as if the device were out of
   // memory, so rollback paths are exercised without exhausting real VRAM.
   void fail_next_granules(int n);
@@ -703,6 +721,8 @@ namespace mi
     std::unique_ptr<DeviceBuffer> staging_;
     // The decode path's split partials and page statistics: this cache's own.
     OwnedWorkspace workspace_;
+    // A chunk's laid-out pages, a stream.
+    StreamBuffers chunk_scratch_;
     // Page statistics kept for fold_kept, every layer's (decode_kept_floats
     // a layer), and the step they belong to.
     OwnedWorkspace kept_;

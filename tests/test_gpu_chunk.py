@@ -1,0 +1,108 @@
+"""A long chunk's attention over laid-out pages (chunk.hip): the sizes where
+its tiles, steps, splits and dispatch end, against the float64 oracle at the
+attention gate (conftest.ATTN_MAX_REL, with the oracle's fp32 error bound)."""
+
+import numpy as np
+import pytest
+
+from conftest import announce, assert_attention_close
+from oracle import attention as att
+from test_gpu_kv_pages import mi, normal, pages_for, put, store_in_runs
+from test_gpu_prefill import P, chunk_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("heads,kv,hd,seq,seq_q,bias", [
+    (32, 8, 64, P * 5 + 3, 63, False),     # the largest chunk that stages page by page
+    (32, 8, 64, P * 5 + 3, 64, False),     # the smallest over laid-out pages
+    (32, 8, 64, 64, 64, False),            # a prompt of whole pages, nothing before it
+    (32, 8, 64, P * 7 + 31, 65, True),     # one query past a workgroup's 64
+    (4, 4, 64, P * 9 + 1, 257, False),     # a head a KV head: 256 queries a workgroup, and one
+    (16, 1, 64, P * 6, 90, False),         # sixteen heads a KV head
+    (14, 2, 64, P * 33 + 17, 73, True),    # rows that do not fill their tiles; steps in splits
+    (12, 2, 128, P * 3 + 2, 64, True),     # head_dim 128: 21 queries a workgroup
+    (12, 2, 128, P * 40 + 30, 150, False),
+    (12, 2, 128, P * 130 + 5, 64, True),   # many splits of few queries
+    (8, 8, 128, P * 4 + 9, 129, False),
+])
+def test_chunks_at_the_edges_of_tiles_and_steps(heads, kv, hd, seq, seq_q, bias):
+    chunk_case(heads, kv, hd, seq, seq_q, 11, bias, True)
+
+
+@pytest.mark.parametrize("hd,kv,heads", [(64, 8, 32), (128, 2, 12)])
+def test_unread_pages_before_and_inside_a_long_chunk(hd, kv, heads):
+    """Masked pages, among them the first, two of one step, and sealed pages
+    of the chunk's own positions."""
+    seq, seq_q = P * 14 + 9, 4 * P
+    chunk_case(heads, kv, hd, seq, seq_q, 3, False, False, (0, 4, 5, 7, 11, 12))
+
+
+@pytest.mark.parametrize("heads,kv,hd", [(32, 8, 64), (12, 2, 128)])
+def test_one_score_far_above_the_rest_moves_the_reference(heads, kv, hd):
+    """Scores that rise by hundreds of powers of two from one page to the
+    next, and fall again: each row's softmax reference moves up step by step
+    and its earlier sums vanish."""
+    rng = np.random.default_rng(2)
+    seq, seq_q = P * 12 + 5, 70
+    k, v = normal(rng, seq, kv, hd), normal(rng, seq, kv, hd)
+    q = normal(rng, seq_q, heads, hd)
+    for page, size in ((1, 4.0), (3, 12.0), (4, 40.0), (8, 6.0)):
+        k[page * P + 7] = size * np.sign(q[0, 0])
+    m = mi()
+    d = m.device
+    alloc, cache = pages_for(P, kv, hd, 0)
+    store_in_runs(cache, 0, k, v, [seq])
+    out = d.empty(q.size)
+    announce("chunk outlier scores", heads, kv, hd)
+    cache.attention(0, put(q), None, None, out, seq_q, seq, heads, kv, hd, None, None, None, None)
+    want, w = att.attention64(q, k, v)
+    assert_attention_close(out.to_numpy().reshape(q.shape), want, "outliers",
+                           att.attention_bound(q, k, v, w))
+
+
+def test_captures_and_further_streams_take_the_staging_path():
+    """A captured launch and a fifth stream get no scratch and take the path
+    that needs none: the same attention, the graph replayed between the
+    program's own calls."""
+    m = mi()
+    d = m.device
+    heads, kv, hd, seq, seq_q = 32, 8, 64, P * 9 + 4, 80
+    rng = np.random.default_rng(9)
+    k, v, q = (normal(rng, seq, kv, hd), normal(rng, seq, kv, hd), normal(rng, seq_q, heads, hd))
+    alloc, cache = pages_for(P, kv, hd, 0)
+    store_in_runs(cache, 0, k, v, [seq])
+    m.synchronize()
+    want, w = att.attention64(q, k, v)
+    bound = att.attention_bound(q, k, v, w)
+    dq, out = put(q), d.empty(q.size)
+    stream = m.Stream()
+
+    def call():
+        cache.attention(0, dq, None, None, out, seq_q, seq, heads, kv, hd, None, None, None, None)
+
+    graph = m.Graph(stream)
+    with graph.capture():
+        call()
+    for i in range(3):
+        announce("chunk graph replay", i)
+        d.random_half(out, 70 + i, 1.0)
+        m.synchronize()
+        graph.launch()
+        stream.synchronize()
+        assert_attention_close(out.to_numpy().reshape(q.shape), want, f"replay {i}", bound)
+        d.random_half(out, 90 + i, 1.0)
+        call()
+        assert_attention_close(out.to_numpy().reshape(q.shape), want, f"eager {i}", bound)
+    streams = [m.Stream() for _ in range(6)]
+    for i, s in enumerate(streams):
+        announce("chunk stream", i)
+        d.random_half(out, i + 1, 1.0)
+        m.synchronize()
+        m.set_stream(s)
+        try:
+            call()
+        finally:
+            m.set_stream(None)
+        s.synchronize()
+        assert_attention_close(out.to_numpy().reshape(q.shape), want, f"stream {i}", bound)
