@@ -463,6 +463,7 @@ namespace mi
   {
     kHalf,       // out fp16 = acc + bias (fp32, one rounding)
     kAccumulate, // out fp32 += acc
+    kFloat,      // out fp32 = acc
     kSwiglu,     // seg[0] gate, seg[1] up: seg[0].out fp16 = silu(g) u
     kLogits,     // out fp32 = acc, and each block's best (value, index)
   };
@@ -504,6 +505,9 @@ namespace mi
     int blocks;
   };
   ProjectPlanInfo launch_project(const ProjectArgs &p, hipStream_t stream);
+  // Whether launch_project takes one row of `in` values at x against the
+  // weights at w: a multiple of 8 values, at most 32768, both 16-byte aligned.
+  bool project_applies(const void *x, const void *w, int in);
   // A step's state in device memory, four ints.
   constexpr int kStepToken = 0;    // the token the step feeds
   constexpr int kStepPosition = 1; // its position

@@ -410,6 +410,9 @@ namespace mi
           *out = *out + dot;
           break;
         }
+        case ProjectMode::kFloat:
+          static_cast<float *>(sg.out)[row] = dot;
+          break;
         case ProjectMode::kSwiglu:
         {
           const float gv = h2f(to_half(dot));
@@ -760,7 +763,8 @@ namespace mi
     // device holds that many workgroups at once -- for gate/up when it
     // holds four fifths of them, the rest a short second round (faster
     // than the resident grid, whose waves hold two rows' registers and so
-    // fit fewer a SIMD); otherwise as many workgroups as it holds,
+    // fit fewer a SIMD; one matrix of 8,960 rows by itself is not: 9.2 us
+    // against the resident grid's 8.0); otherwise as many workgroups as it holds,
     // each wave over several rows with the next row's runs in flight while
     // one is used.
     ProjectPlan plan_projection(const ProjectArgs &p)
@@ -801,6 +805,12 @@ namespace mi
       return {pipe, waves, static_cast<int>(std::min<long long>(needed, held)), lds, split, true};
     }
   } // namespace
+
+  bool project_applies(const void *x, const void *w, int in)
+  {
+    return in > 0 && in % 8 == 0 && in <= 32768 &&
+           (reinterpret_cast<std::uintptr_t>(x) | reinterpret_cast<std::uintptr_t>(w)) % 16 == 0;
+  }
 
   int project_blocks(const ProjectArgs &p)
   {
