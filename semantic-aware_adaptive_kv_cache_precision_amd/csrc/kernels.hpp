@@ -146,6 +146,19 @@ namespace mi
   void launch_row_jobs(const RowJob *jobs, int count, int page_tokens, int kv_heads, int head_dim,
                        hipStream_t stream);
 
+  // Whole pages of consecutive positions, sealed from a store's own rows: page
+  // i's keys and values are rows 32 i .. 32 i + 31 of `keys` and `values`,
+  // its place and tier dst[i] (the tier in the low 4 bits of an address that
+  // page slots keep zero). One launch takes kRowRunPages of them where
+  // launch_row_jobs takes kRowJobsALaunch: a 2,048-row chunk's 64 pages in
+  // one launch of 9 us, not three of 8. Shapes of the register quantiser
+  // (row_run_applies); others go through launch_row_jobs.
+  constexpr int kRowRunPages = 256;
+  bool row_run_applies(int page_tokens, int kv_heads, int head_dim);
+  void launch_row_run(const std::uint16_t *keys, const std::uint16_t *values,
+                      const unsigned long long *dst, int count, int kv_heads, int head_dim,
+                      hipStream_t stream);
+
   // Page table edits: entry `index` of the address and tier arrays set.
   struct TableEdit
   {

@@ -466,6 +466,14 @@ namespace mi
     const int first_span = start / page_tokens_;
     const int end = start + n;
     std::vector<RowJob> jobs;
+    // Whole pages of the store's own rows, consecutive: their places and
+    // tiers, and the first one's first row.
+    std::vector<unsigned long long> run;
+    int run_first = 0;
+    const std::uint16_t *run_keys = nullptr;
+    const std::uint16_t *run_values = nullptr;
+    const bool runs = halves_ == Halves::kBoth && n > 2 * page_tokens_ &&
+                      row_run_applies(page_tokens_, kv_heads_, head_dim_);
     for (int span = first_span; span * page_tokens_ < end; ++span)
     {
       const int span_start = span * page_tokens_;
@@ -480,6 +488,20 @@ namespace mi
         // page holds before `a` and the rows brought from `a` on.
         const PageKey key{layer, span};
         const PageLocation at = allocator_.locate(key);
+        const auto place = reinterpret_cast<unsigned long long>(allocator_.address_of(at));
+        if (runs && a == span_start && place % 16 == 0 &&
+            (run.empty() || span == run_first + static_cast<int>(run.size())))
+        {
+          if (run.empty())
+          {
+            run_first = span;
+            run_keys = k_rows;
+            run_values = v_rows;
+          }
+          run.push_back(place | static_cast<unsigned long long>(at.tier));
+          sealed_[layer] = std::max(sealed_[layer], span + 1);
+          continue;
+        }
         const std::uint16_t *open = open_page(layer, cur);
         j.k_lo = open;
         j.v_lo = open + half;
@@ -519,8 +541,16 @@ namespace mi
       }
       jobs.push_back(j);
     }
-    launch_row_jobs(jobs.data(), static_cast<int>(jobs.size()), page_tokens_, kv_heads_,
-                    head_dim_, runtime_stream());
+    if (!run.empty())
+    {
+      launch_row_run(run_keys, run_values, run.data(), static_cast<int>(run.size()), kv_heads_,
+                     head_dim_, runtime_stream());
+    }
+    if (!jobs.empty())
+    {
+      launch_row_jobs(jobs.data(), static_cast<int>(jobs.size()), page_tokens_, kv_heads_,
+                      head_dim_, runtime_stream());
+    }
   }
 
   // ---- evict, mask ---------------------------------------------------------------------

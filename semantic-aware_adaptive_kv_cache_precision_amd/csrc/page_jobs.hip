@@ -261,6 +261,35 @@ namespace mi
       run_row_task<HD>(jobs.job[blockIdx.y], jobs.lay, task, kv_heads);
     }
 
+    struct RowRun
+    {
+      const std::uint16_t *keys;
+      const std::uint16_t *values;
+      unsigned long long dst[kRowRunPages];
+      PageLayout lay[kTierCount];
+    };
+
+    // Page blockIdx.y of the run, tasks blockIdx.x * 256 + tid (of W).
+    template <int HD>
+    __global__ void __launch_bounds__(kThreads) row_run_kernel(RowRun r, int kv_heads)
+    {
+      const int task = blockIdx.x * kThreads + threadIdx.x;
+      const int W = kv_heads * HD;
+      if (task >= W)
+      {
+        return;
+      }
+      const std::size_t first = static_cast<std::size_t>(blockIdx.y) * kP * W;
+      const unsigned long long dst = r.dst[blockIdx.y];
+      RowJob j{};
+      j.tier = static_cast<int>(dst & 15);
+      j.kind = static_cast<int>(j.tier == kFP16 ? RowJobKind::kCopy : RowJobKind::kQuantise);
+      j.k_lo = j.k_hi = r.keys + first;
+      j.v_lo = j.v_hi = r.values + first;
+      j.dst = reinterpret_cast<std::uint8_t *>(dst - (dst & 15));
+      run_row_task<HD>(j, r.lay, task, kv_heads);
+    }
+
     // A decode step's store, its position read on the device: the one row
     // fills row position % P of the open page, or, on a page's last row,
     // the page is sealed from the open page's rows and this one.
@@ -597,6 +626,42 @@ namespace mi
       hip_check(hipGetLastError(), "quantise (registers) kernel launch");
     });
     return true;
+  }
+
+  bool row_run_applies(int page_tokens, int kv_heads, int head_dim)
+  {
+    return register_shape(page_tokens, kv_heads, head_dim);
+  }
+
+  void launch_row_run(const std::uint16_t *keys, const std::uint16_t *values,
+                      const unsigned long long *dst, int count, int kv_heads, int head_dim,
+                      hipStream_t stream)
+  {
+    RowRun run{};
+    for (int t = kINT8; t <= kINT2; ++t)
+    {
+      run.lay[t] = page_layout(t, kP, kv_heads, head_dim);
+    }
+    const std::size_t W = static_cast<std::size_t>(kv_heads) * head_dim;
+    const int blocks = static_cast<int>((W + kThreads - 1) / kThreads);
+    for (int first = 0; first < count; first += kRowRunPages)
+    {
+      const int n = std::min(kRowRunPages, count - first);
+      run.keys = keys + static_cast<std::size_t>(first) * kP * W;
+      run.values = values + static_cast<std::size_t>(first) * kP * W;
+      std::copy(dst + first, dst + first + n, run.dst);
+      if (head_dim == 128)
+      {
+        hipLaunchKernelGGL(row_run_kernel<128>, dim3(blocks, n), dim3(kThreads), 0, stream, run,
+                           kv_heads);
+      }
+      else
+      {
+        hipLaunchKernelGGL(row_run_kernel<64>, dim3(blocks, n), dim3(kThreads), 0, stream, run,
+                           kv_heads);
+      }
+      hip_check(hipGetLastError(), "row run kernel launch");
+    }
   }
 
   void launch_row_jobs(const RowJob *jobs, int count, int page_tokens, int kv_heads, int head_dim,
