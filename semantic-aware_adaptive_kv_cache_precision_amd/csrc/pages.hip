@@ -81,13 +81,30 @@ namespace mi
       {
         return;
       }
+      // The masses and the old score in one trip, eight heads at a time.
+      const float old = scores[page];
       float total = 0.0f;
       const float *column = mass + page;
-      for (int h = 0; h < heads; ++h, column += pages)
+      int h = 0;
+      for (; h + 8 <= heads; h += 8, column += 8 * static_cast<std::size_t>(pages))
+      {
+        float m[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+        {
+          m[i] = column[i * static_cast<std::size_t>(pages)];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+        {
+          total = __fadd_rn(total, m[i]);
+        }
+      }
+      for (; h < heads; ++h, column += pages)
       {
         total = __fadd_rn(total, *column);
       }
-      scores[page] = ewma_step(scores[page], __fdiv_rn(total, static_cast<float>(heads)), alpha);
+      scores[page] = ewma_step(old, __fdiv_rn(total, static_cast<float>(heads)), alpha);
     }
 
     int grid_for(std::size_t count, int threads, int cap = 65536)
