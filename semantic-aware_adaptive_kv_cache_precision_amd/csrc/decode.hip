@@ -76,6 +76,20 @@ namespace mi
     constexpr int kPageTokens = 32;
     constexpr int kMaxGroup = 16;
     constexpr int kMaxHeads = 64;
+    // Pages a split of one layer's launch takes, a wave each: half a
+    // workgroup's waves where the launch then still has no more workgroups
+    // than the device has CUs, so that a wave has a SIMD to itself (the rest
+    // of the workgroup idles); otherwise all of them. 28 layers at 4,999
+    // positions of the 1.5B shape with the key bias: 438 -> 382 us a token,
+    // at 15,000 (236 workgroups) 445 -> 400; at 32,768, where halving the
+    // pages would double the workgroups past the CUs, 403 -> 496.
+    __host__ __device__ inline int split_pages_of(int pages, int kv_heads, int cus)
+    {
+      return static_cast<long long>((pages + kWaves / 2 - 1) / (kWaves / 2)) * kv_heads <= cus
+                 ? kWaves / 2
+                 : kWaves;
+    }
+
     constexpr int kOwnPage = 0xFE; // the query's own page: open page + chunk rows
 
     struct DecodeArgs
@@ -112,6 +126,10 @@ namespace mi
       int pages;
       int pages_per_wave;
       int splits;
+      // Waves of a split's workgroup that take pages (split_pages_of), and
+      // the device's CUs, by which a live launch chooses it.
+      int split_waves;
+      int cus;
       float scale; // 1/sqrt(hd) * log2 e: scores in base-2 units
       // Streaming launches: the (layer, KV-head block, page) units split into
       // stream_ranges equal contiguous ranges. A range is walked by
@@ -206,8 +224,8 @@ namespace mi
         a.seq_k = seq_k;
         a.start = seq_k - 1;
         a.live_pages = (seq_k + kPageTokens - 1) / kPageTokens;
-        const int per_split = kWaves * a.pages_per_wave;
-        a.live_splits = (a.live_pages + per_split - 1) / per_split;
+        a.split_waves = split_pages_of(a.live_pages, a.value_kv_heads, a.cus);
+        a.live_splits = (a.live_pages + a.split_waves - 1) / a.split_waves;
       }
     }
 
@@ -904,16 +922,18 @@ namespace mi
       const unsigned long long *table = a.table + layer * a.table_stride;
       const std::uint8_t *tiers = a.tiers != nullptr ? a.tiers + layer * a.table_stride : nullptr;
       const int own = a.causal ? (a.seq_k - 1) / kPageTokens : -1;
-      const int p0 = (split * kWaves + wave) * a.pages_per_wave;
+      const int p0 = wave < a.split_waves
+                         ? (split * a.split_waves + wave) * a.pages_per_wave
+                         : a.live_pages; // an idle wave: no pages
       // The wave's pages: p0 and the next pages_per_wave - 1 (several a
-      // wave), or p0 and every kWaves * busy pages on (the pages past the
+      // wave), or p0 and every split_waves * busy pages on (the pages past the
       // busy splits).
       int p_step = 1, p_count = a.pages_per_wave, p_bound = a.live_pages;
       if constexpr (!kBias)
       {
         if (a.pages_per_wave == 1)
         {
-          p_step = kWaves * busy;
+          p_step = a.split_waves * busy;
           p_count = INT_MAX;
         }
       }
@@ -2470,6 +2490,8 @@ namespace mi
     d.value_kv_heads = a.kv_heads;
     d.stat_group = group;
     d.pages = pages;
+    d.cus = device_multiprocessors();
+    d.split_waves = kWaves;
     // Scores in base-2 units: the softmax weights are exp2 of them.
     d.scale = static_cast<float>(1.4426950408889634 / std::sqrt(static_cast<double>(a.head_dim)));
     // One layer: a page a wave, so a launch has a wave for every page of
@@ -2551,8 +2573,12 @@ namespace mi
     }
     else if (ls.split)
     {
+      // (A live launch may see fewer pages: `splits` holds the most any
+      // count up to `pages` makes, in every launch, so that kept statistics
+      // have one layout.)
       d.pages_per_wave = 1;
-      d.splits = (pages + kWaves - 1) / kWaves;
+      d.splits = decode_splits(a.kv_heads, pages);
+      d.split_waves = split_pages_of(pages, a.kv_heads, d.cus);
     }
     else
     {
@@ -2560,7 +2586,7 @@ namespace mi
       d.splits = 1;
     }
     d.live_pages = pages;
-    d.live_splits = d.splits;
+    d.live_splits = ls.split && !streaming ? (pages + d.split_waves - 1) / d.split_waves : d.splits;
     // head_dim 64 with an even number of KV heads and no key bias (the
     // Llama shapes): two KV heads a wave, as one 128-channel unit, so that a
     // launch has half the waves, each with a unit of the size the kernel's
@@ -2628,13 +2654,13 @@ namespace mi
         // One layer split a page a wave (no key bias): no more workgroups a
         // KV head than the device holds at once (past that, second pages
         // for some waves).
-        int grid_splits = d.splits;
+        int grid_splits = d.live_seq_k != nullptr ? d.splits : d.live_splits;
         if (ls.split && d.k_bias == nullptr)
         {
           const long long per = resident_pages_blocks(reinterpret_cast<const void *>(pages_kernel),
                                                       lds) /
                                 (static_cast<long long>(d.kv_heads) * ls.layers);
-          if (per < d.splits)
+          if (per < grid_splits)
           {
             d.busy_splits = static_cast<int>(std::max<long long>(per, 1));
             grid_splits = d.busy_splits;
@@ -2705,11 +2731,18 @@ namespace mi
     }
   }
 
+  int decode_splits(int kv_heads, int pages)
+  {
+    constexpr int kHalf = kWaves / 2;
+    const int most_halved = device_multiprocessors() / kv_heads; // workgroups a KV head
+    return std::max((pages + kWaves - 1) / kWaves,
+                    std::min((pages + kHalf - 1) / kHalf, most_halved));
+  }
+
   std::size_t decode_kept_floats(int heads, int kv_heads, int seq_k)
   {
     const int pages = (seq_k + kPageTokens - 1) / kPageTokens;
-    const int splits = (pages + kWaves - 1) / kWaves;
-    (void)kv_heads;
+    const int splits = decode_splits(kv_heads, pages);
     return static_cast<std::size_t>(heads) * splits * 2 + static_cast<std::size_t>(heads) * pages * 2;
   }
 
@@ -2728,7 +2761,9 @@ namespace mi
     d.stat_group = d.group;
     d.pages = pages;
     d.seq_k = f.seq_k;
-    d.splits = (pages + kWaves - 1) / kWaves;
+    d.splits = decode_splits(f.kv_heads, pages);
+    d.cus = device_multiprocessors();
+    d.split_waves = split_pages_of(pages, f.kv_heads, d.cus);
     d.split_ml = f.kept;
     d.page_stats = f.kept + static_cast<std::size_t>(f.layers) * f.heads * d.splits * 2;
     d.mass = f.mass;
@@ -2738,7 +2773,7 @@ namespace mi
     d.alpha = f.alpha;
     d.live_seq_k = f.live_seq_k;
     d.live_pages = pages;
-    d.live_splits = d.splits;
+    d.live_splits = (pages + d.split_waves - 1) / d.split_waves;
     d.pages_per_wave = 1;
     d.score_every = std::max(1, f.score_every);
     d.mass_blocks = (pages + 63) / 64;

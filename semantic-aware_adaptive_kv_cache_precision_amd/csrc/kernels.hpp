@@ -436,6 +436,9 @@ namespace mi
   // pages, head_dim 64 or 128, a group of at most 16 heads, 16-byte aligned
   // rows and page regions.
   bool decode_fast_applies(const KVSource &kv, const AttentionArgs &a);
+  // The most splits a KV head of a one-layer launch makes over any number of
+  // pages up to `pages`: the stride of its per-split arrays.
+  int decode_splits(int kv_heads, int pages);
   void launch_decode_layers(const KVSource &kv, const AttentionArgs &a, const DecodeLayers &ls,
                             hipStream_t stream);
 

@@ -1370,7 +1370,7 @@ namespace mi
     // The split decode's partials, split maxima and page statistics at
     // max_seq_k (the largest launch of the run).
     const int pages = (max_seq_k + page_tokens_ - 1) / page_tokens_;
-    const int splits = (pages + 7) / 8;
+    const int splits = decode_splits(kv_heads_, pages);
     workspace_.floats(static_cast<std::size_t>(heads) * splits * (head_dim + 2) +
                       static_cast<std::size_t>(heads) * pages * 2);
   }

@@ -1,0 +1,86 @@
+"""One layer's decode where its split changes: half a workgroup's waves a
+split up to a workgroup a CU, all of them past it. Outputs and masses against
+the float64 oracle on both sides; a launch sized for a long context with its
+seq_k on the device, and the statistics kept for a later fold, to the bits of
+the plain launch at every seq_k."""
+
+import numpy as np
+import pytest
+
+from conftest import announce, assert_attention_close, fp16_exact
+from oracle import attention as att
+from oracle import ewma
+from test_gpu_kv_pages import LAYERS, mi, normal, page_sizes, put, sealed_pages
+
+pytestmark = pytest.mark.gpu
+
+P = 32
+THETA = 1e6
+
+
+def cache_of(seq, kv, hd, most):
+    m = mi()
+    pages = most // P + 1
+    tmap = [[(1, 0, 3, 2)[(p + l) % 4] for p in range(pages)] for l in range(LAYERS)]
+    cap = [pages * LAYERS + 16] * 4
+    alloc = m.PagedKVCache(page_sizes(P, kv, hd), cap)
+    cache = m.device.KVPages(alloc, LAYERS, P, kv, hd, 0, m.device.Halves.Both, tmap, True)
+    cache.reserve(most)
+    return alloc, cache
+
+
+@pytest.mark.parametrize("heads,kv,hd,bias", [(12, 2, 128, False), (12, 2, 128, True),
+                                              (14, 2, 64, True), (32, 8, 64, False),
+                                              (5, 1, 128, False)])
+def test_decode_on_both_sides_of_the_split(heads, kv, hd, bias):
+    m = mi()
+    d = m.device
+    # The pages at which halved splits would pass a workgroup a CU (256 CUs).
+    edge = 256 // kv * 4 * P
+    most = edge + 3 * P
+    rng = np.random.default_rng(heads + hd + bias)
+    k, v = normal(rng, most, kv, hd), normal(rng, most, kv, hd)
+    b = fp16_exact(3 * rng.standard_normal((kv, hd))) if bias else None
+    db = put(b) if bias else None
+    rope = d.RopeTable(hd, THETA) if bias else None
+    if bias:
+        rope.cover(most)
+    part = d.empty_f32(d.attention_partials(hd))
+    q = [put(normal(rng, heads, hd)) for _ in range(LAYERS)]
+    for seq in (1, P + 1, 5 * P, edge, edge + 1, edge + 2 * P + 7):
+        alloc, cache = cache_of(seq, kv, hd, most)
+        for l in range(LAYERS):
+            if seq > 1:
+                cache.store(l, put(k[:seq - 1]), put(v[:seq - 1]), 0, seq - 1)
+            cache.store(l, put(k[seq - 1:seq]), put(v[seq - 1:seq]), seq - 1, 1)
+        kr, vr = put(k[seq - 1:seq]), put(v[seq - 1:seq])
+        pages = -(-seq // P)
+        masses, outs = [], []
+        for l in range(LAYERS):
+            announce("decode", heads, kv, hd, "bias" if bias else "", seq, l)
+            out, mass = d.empty(heads * hd), d.empty_f32(heads * pages)
+            cache.attention(l, q[l], db, rope, out, 1, seq, heads, kv, hd, kr, vr, mass, part)
+            outs.append(out.raw())
+            masses.append(mass.to_numpy())
+            live = d.empty(heads * hd)
+            cache.attention_at(l, q[l], db, rope, live, d.DeviceIndex([seq]), most, heads, kv, hd,
+                               kr, vr)
+            np.testing.assert_array_equal(live.raw().view(np.uint16), outs[l].view(np.uint16))
+        kept = d.empty(heads * hd)
+        for l in range(LAYERS):
+            cache.attention_kept(l, q[l], db, rope, kept, seq, heads, kv, hd, kr, vr)
+            np.testing.assert_array_equal(kept.raw().view(np.uint16), outs[l].view(np.uint16))
+        scores = d.ImportanceScores(LAYERS, pages)
+        mass = d.empty_f32(LAYERS * heads * pages)
+        cache.fold_kept(scores=scores, mass=mass, seq_k=seq, heads=heads)
+        got = mass.to_numpy().reshape(LAYERS, heads, pages)
+        np.testing.assert_array_equal(got, np.stack(masses).reshape(got.shape))
+        np.testing.assert_array_equal(
+            scores.download(), ewma.host_ewma([(l, got[l]) for l in range(LAYERS)], LAYERS, pages))
+        sealed, tiers = sealed_pages(alloc, 0, (seq - 1) // P)
+        want, bound = att.causal_chunk(q[0].raw().reshape(1, heads, hd).astype(np.float32), sealed,
+                                       tiers, k[:seq], v[:seq], kv, hd, P, b, THETA,
+                                       with_bound=True)
+        assert_attention_close(outs[0].astype(np.float64).reshape(1, heads, hd), want,
+                               f"seq {seq}", bound)
+        np.testing.assert_allclose(got[0].sum(1), 1.0, rtol=1e-3)
