@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import ctypes as C
 import enum
+import functools
 import os
 import weakref
 from pathlib import Path
@@ -651,6 +652,15 @@ def _need(span, count: int, what: str) -> int:
     return span.address
 
 
+def _at(x, count: int, what: str) -> int:
+    """The address of a tensor or view that must hold `count` elements:
+    _need of its span, without making one."""
+    held = x.count if isinstance(x, Span) else x.numel
+    if held < count:
+        raise ValueError(f"{what} holds {held}, and the operation needs {count}")
+    return x.address
+
+
 def _non_negative(value: int, what: str) -> None:
     if value < 0:
         raise ValueError(f"{what} must not be negative, got {value}")
@@ -694,6 +704,7 @@ class DeviceIndex:
         return self._storage.ptr
 
 
+@functools.lru_cache(maxsize=64)
 def _attention_partials(head_dim: int) -> int:
     return int(lib.mi_attention_partials_floats(head_dim))
 
@@ -761,15 +772,18 @@ class ImportanceScores:
         _check(lib.mi_scores_create(layers, max_pages, alpha, C.byref(h)))
         self._h = h.value
         weakref.finalize(self, lib.mi_scores_destroy, self._h)
+        # What a decode call asks for every time and never changes.
+        self._layers, self._max_pages, self._alpha, _ = self._info()
+        self._rows = {}
 
     def _info(self):
         l, m, a, d = C.c_int(), C.c_int(), C.c_float(), C.c_size_t()
         _check(lib.mi_scores_info(self._h, C.byref(l), C.byref(m), C.byref(a), C.byref(d)))
         return l.value, m.value, a.value, d.value
 
-    layers = property(lambda self: self._info()[0])
-    max_pages = property(lambda self: self._info()[1])
-    alpha = property(lambda self: self._info()[2])
+    layers = property(lambda self: self._layers)
+    max_pages = property(lambda self: self._max_pages)
+    alpha = property(lambda self: self._alpha)
     downloads = property(lambda self: self._info()[3])
 
     @property
@@ -779,9 +793,12 @@ class ImportanceScores:
 
     def row(self, layer: int) -> int:
         """The device address of a layer's scores, for a fused fold."""
-        p = _vp()
-        _check(lib.mi_scores_layer_row(self._h, layer, C.byref(p)))
-        return p.value
+        at = self._rows.get(layer)
+        if at is None:
+            p = _vp()
+            _check(lib.mi_scores_layer_row(self._h, layer, C.byref(p)))
+            at = self._rows[layer] = p.value
+        return at
 
     def fold(self, layer: int, mass: FloatTensor, heads: int, pages: int) -> None:
         if heads > 0 and pages > 0 and mass.numel < heads * pages:
@@ -965,6 +982,10 @@ class KVPages:
         self._h = h.value
         self._allocator = allocator
         weakref.finalize(self, lib.mi_kv_destroy, self._h)
+        # The cache's shape, which calls check their operands against.
+        info = self._info()
+        self._layers, self._page_tokens, self._kv_width = (info.layers, info.page_tokens,
+                                                           info.kv_width)
 
     @staticmethod
     def seals_for(tier, tier_map=None, always_seal=False) -> bool:
@@ -979,12 +1000,12 @@ class KVPages:
         _check(lib.mi_kv_info_get(self._h, C.byref(info)))
         return info
 
-    page_tokens = property(lambda self: self._info().page_tokens)
+    page_tokens = property(lambda self: self._page_tokens)
+    layers = property(lambda self: self._layers)
+    kv_width = property(lambda self: self._kv_width)
     pages_per_layer = property(lambda self: self._info().pages_per_layer)
-    layers = property(lambda self: self._info().layers)
     capacity_tokens = property(lambda self: self._info().capacity_tokens)
     page_bytes = property(lambda self: self._info().page_bytes)
-    kv_width = property(lambda self: self._info().kv_width)
     tier = property(lambda self: Tier(self._info().tier))
     halves = property(lambda self: Halves(self._info().halves))
     storage_tier = property(lambda self: Tier(self._info().storage_tier))
@@ -999,8 +1020,8 @@ class KVPages:
     def store(self, layer: int, keys, values, start: int, n: int) -> None:
         _non_negative(n, "n")
         width = self.kv_width
-        k = _need(_span(keys), n * width, "keys")
-        v = _need(_span(values), n * width, "values")
+        k = _at(keys, n * width, "keys")
+        v = _at(values, n * width, "values")
         _check(lib.mi_kv_store(self._h, layer, k, v, start, n))
 
     def attention(self, layer: int, q, k_bias, rope, out, seq_q: int, seq_k: int, heads: int,
@@ -1012,11 +1033,11 @@ class KVPages:
         if seq_q > seq_k:
             raise ValueError(f"seq_q {seq_q} exceeds seq_k {seq_k}")
         _non_negative(seq_q, "seq_q")
-        qa = _need(_span(q), seq_q * heads * head_dim, "q")
-        oa = _need(_span(out), seq_q * heads * head_dim, "out")
-        ba = _need(_span(k_bias), kv_heads * head_dim, "k_bias") if k_bias is not None else None
-        ka = _need(_span(keys), seq_q * kv_heads * head_dim, "keys") if keys is not None else None
-        va = (_need(_span(values), seq_q * kv_heads * head_dim, "values")
+        qa = _at(q, seq_q * heads * head_dim, "q")
+        oa = _at(out, seq_q * heads * head_dim, "out")
+        ba = _at(k_bias, kv_heads * head_dim, "k_bias") if k_bias is not None else None
+        ka = _at(keys, seq_q * kv_heads * head_dim, "keys") if keys is not None else None
+        va = (_at(values, seq_q * kv_heads * head_dim, "values")
               if values is not None else None)
         P = self.page_tokens
         pages = -(-seq_k // P)
@@ -1049,10 +1070,10 @@ class KVPages:
         _non_negative(layers, "layers")
         per_q = heads * head_dim
         width = kv_heads * head_dim
-        qa = _need(_span(q), layers * per_q, "q")
-        oa = _need(_span(out), layers * per_q, "out")
-        ka = _need(_span(keys), layers * width, "keys") if keys is not None else None
-        va = _need(_span(values), layers * width, "values") if values is not None else None
+        qa = _at(q, layers * per_q, "q")
+        oa = _at(out, layers * per_q, "out")
+        ka = _at(keys, layers * width, "keys") if keys is not None else None
+        va = _at(values, layers * width, "values") if values is not None else None
         pages = -(-seq_k // self.page_tokens)
         ma = None
         if mass is not None:
@@ -1076,11 +1097,11 @@ class KVPages:
         layer's masses and folds them into the scores in one launch."""
         per_q = heads * head_dim
         width = kv_heads * head_dim
-        qa = _need(_span(q), per_q, "q")
-        oa = _need(_span(out), per_q, "out")
-        ba = _need(_span(k_bias), width, "k_bias") if k_bias is not None else None
-        ka = _need(_span(keys), width, "keys") if keys is not None else None
-        va = _need(_span(values), width, "values") if values is not None else None
+        qa = _at(q, per_q, "q")
+        oa = _at(out, per_q, "out")
+        ba = _at(k_bias, width, "k_bias") if k_bias is not None else None
+        ka = _at(keys, width, "keys") if keys is not None else None
+        va = _at(values, width, "values") if values is not None else None
         _check(lib.mi_kv_attention_kept(self._h, layer, qa, ba, rope._h if rope else None, oa,
                                         seq_k, heads, kv_heads, head_dim, ka, va))
 
@@ -1089,8 +1110,8 @@ class KVPages:
         held in device memory (`position`, one int), read when the kernel
         runs; the row that completes a page seals it."""
         width = self.kv_width
-        _check(lib.mi_kv_store_at(self._h, layer, _need(_span(keys), width, "keys"),
-                                  _need(_span(values), width, "values"), position.address))
+        _check(lib.mi_kv_store_at(self._h, layer, _at(keys, width, "keys"),
+                                  _at(values, width, "values"), position.address))
 
     def attention_at(self, layer: int, q, k_bias, rope, out, seq_k: DeviceIndex, max_seq_k: int,
                      heads: int, kv_heads: int, head_dim: int, keys, values) -> None:
@@ -1099,12 +1120,12 @@ class KVPages:
         attention(..., partials) at that seq_k."""
         per_q = heads * head_dim
         width = kv_heads * head_dim
-        ba = _need(_span(k_bias), width, "k_bias") if k_bias is not None else None
-        _check(lib.mi_kv_attention_at(self._h, layer, _need(_span(q), per_q, "q"), ba,
-                                      rope._h if rope else None, _need(_span(out), per_q, "out"),
+        ba = _at(k_bias, width, "k_bias") if k_bias is not None else None
+        _check(lib.mi_kv_attention_at(self._h, layer, _at(q, per_q, "q"), ba,
+                                      rope._h if rope else None, _at(out, per_q, "out"),
                                       seq_k.address, max_seq_k, heads, kv_heads, head_dim,
-                                      _need(_span(keys), width, "keys"),
-                                      _need(_span(values), width, "values")))
+                                      _at(keys, width, "keys"),
+                                      _at(values, width, "values")))
 
     def rope_store(self, layer: int, qk, qk_out, q_heads: int, position: DeviceIndex,
                    rope: "RopeTable", values, norm=None) -> None:
@@ -1117,8 +1138,8 @@ class KVPages:
         rmsnorm_f32, rope_from_table and store."""
         width = self.kv_width
         rows = q_heads * rope.head_dim + width
-        qa = _need(_span(qk), rows, "qk")
-        oa = _need(_span(qk_out), rows, "qk_out")
+        qa = _at(qk, rows, "qk")
+        oa = _at(qk_out, rows, "qk_out")
         if qa == oa:
             raise ValueError("rope cannot write over its input")
         if position.count < 1:
@@ -1129,10 +1150,10 @@ class KVPages:
             x, weight, out, eps = norm
             hidden = x.numel
             xa = x.address
-            wa = _need(_span(weight), hidden, "norm weight")
-            na = _need(_span(out), hidden, "normed")
+            wa = _at(weight, hidden, "norm weight")
+            na = _at(out, hidden, "normed")
         _check(lib.mi_kv_rope_store(self._h, layer, qa, oa, q_heads, position.address, rope._h,
-                                    _need(_span(values), width, "values"), xa, wa, na, hidden,
+                                    _at(values, width, "values"), xa, wa, na, hidden,
                                     float(eps)))
 
     def attend_row(self, layer: int, qk, qk_out, q_heads: int, seq_k: int, rope: "RopeTable",
@@ -1146,8 +1167,8 @@ class KVPages:
         width = self.kv_width
         hd = rope.head_dim
         rows = q_heads * hd + width
-        qa = _need(_span(qk), rows, "qk")
-        oa = _need(_span(qk_out), rows, "qk_out") if qk_out is not None else None
+        qa = _at(qk, rows, "qk")
+        oa = _at(qk_out, rows, "qk_out") if qk_out is not None else None
         if qa == oa:
             raise ValueError("rope cannot write over its input")
         xa = wa = na = None
@@ -1156,11 +1177,11 @@ class KVPages:
             x, weight, normed, eps = norm
             hidden = x.numel
             xa = x.address
-            wa = _need(_span(weight), hidden, "norm weight")
-            na = _need(_span(normed), hidden, "normed")
+            wa = _at(weight, hidden, "norm weight")
+            na = _at(normed, hidden, "normed")
         _check(lib.mi_kv_attend_row(self._h, layer, qa, oa, q_heads, seq_k, rope._h,
-                                    _need(_span(values), width, "values"),
-                                    _need(_span(out), q_heads * hd, "out"), xa, wa, na, hidden,
+                                    _at(values, width, "values"),
+                                    _at(out, q_heads * hd, "out"), xa, wa, na, hidden,
                                     float(eps)))
 
     def stored_on_device(self, end: int) -> None:
@@ -1285,11 +1306,11 @@ def _device_attention(q, k, v, k_bias, rope_table, out, seq_q, seq_k, heads, kv_
                       partials=None):
     if seq_q > seq_k:
         raise ValueError(f"seq_q {seq_q} exceeds seq_k {seq_k}")
-    qa = _need(_span(q), seq_q * heads * head_dim, "q")
-    ka = _need(_span(k), seq_k * kv_heads * head_dim, "k")
-    va = _need(_span(v), seq_k * kv_heads * head_dim, "v")
-    ba = _need(_span(k_bias), kv_heads * head_dim, "k_bias") if k_bias is not None else None
-    oa = _need(_span(out), seq_q * heads * head_dim, "out")
+    qa = _at(q, seq_q * heads * head_dim, "q")
+    ka = _at(k, seq_k * kv_heads * head_dim, "k")
+    va = _at(v, seq_k * kv_heads * head_dim, "v")
+    ba = _at(k_bias, kv_heads * head_dim, "k_bias") if k_bias is not None else None
+    oa = _at(out, seq_q * heads * head_dim, "out")
     pa = _floats(partials, _attention_partials(head_dim), "attention's partials")
     data = rope_table._data() if rope_table is not None else None
     positions = rope_table.positions if rope_table is not None else 0
@@ -1301,25 +1322,25 @@ def _device_attention(q, k, v, k_bias, rope_table, out, seq_q, seq_k, heads, kv_
 
 
 def _device_rmsnorm(x, weight, out, rows, hidden, eps):
-    xa = _need(_span(x), rows * hidden, "x")
-    wa = _need(_span(weight), hidden, "weight")
-    oa = _need(_span(out), rows * hidden, "out")
+    xa = _at(x, rows * hidden, "x")
+    wa = _at(weight, hidden, "weight")
+    oa = _at(out, rows * hidden, "out")
     _check(lib.mi_rmsnorm(xa, 0, wa, oa, rows, hidden, eps, None))
 
 
 def _device_rmsnorm_f32(x: FloatTensor, weight, out, rows, hidden, eps):
     if x.numel < rows * hidden:
         raise ValueError(f"x holds {x.numel}, and the operation needs {rows * hidden}")
-    wa = _need(_span(weight), hidden, "weight")
-    oa = _need(_span(out), rows * hidden, "out")
+    wa = _at(weight, hidden, "weight")
+    oa = _at(out, rows * hidden, "out")
     _check(lib.mi_rmsnorm(x.address, 1, wa, oa, rows, hidden, eps, None))
 
 
 def _device_rope(x, positions: DeviceIndex, out, seq, heads, head_dim, theta):
-    xa = _need(_span(x), seq * heads * head_dim, "x")
+    xa = _at(x, seq * heads * head_dim, "x")
     if positions.count < seq:
         raise ValueError(f"positions holds {positions.count}, and the operation needs {seq}")
-    oa = _need(_span(out), seq * heads * head_dim, "out")
+    oa = _at(out, seq * heads * head_dim, "out")
     if xa == oa:
         raise ValueError("rope cannot write over its input")
     _check(lib.mi_rope(xa, positions.address, oa, seq, heads, head_dim, theta, None))
@@ -1329,10 +1350,10 @@ def _device_rope_from_table(x, positions: DeviceIndex, table: "RopeTable", out, 
                             head_dim):
     """_device_rope's rows with the angles read from `table` (beyond the
     reference): every position must be below table.positions."""
-    xa = _need(_span(x), seq * heads * head_dim, "x")
+    xa = _at(x, seq * heads * head_dim, "x")
     if positions.count < seq:
         raise ValueError(f"positions holds {positions.count}, and the operation needs {seq}")
-    oa = _need(_span(out), seq * heads * head_dim, "out")
+    oa = _at(out, seq * heads * head_dim, "out")
     if xa == oa:
         raise ValueError("rope cannot write over its input")
     if table.head_dim != head_dim:
@@ -1343,51 +1364,51 @@ def _device_rope_from_table(x, positions: DeviceIndex, table: "RopeTable", out, 
 
 
 def _device_swiglu(gate, up, out, count):
-    ga = _need(_span(gate), count, "gate")
-    ua = _need(_span(up), count, "up")
-    oa = _need(_span(out), count, "out")
+    ga = _at(gate, count, "gate")
+    ua = _at(up, count, "up")
+    oa = _at(out, count, "out")
     if oa in (ga, ua):
         raise ValueError("swiglu cannot write over its input")
     _check(lib.mi_swiglu(ga, ua, oa, count, None))
 
 
 def _device_add(a, b, out, count):
-    _check(lib.mi_add(_need(_span(a), count, "a"), _need(_span(b), count, "b"),
-                      _need(_span(out), count, "out"), count, None))
+    _check(lib.mi_add(_at(a, count, "a"), _at(b, count, "b"),
+                      _at(out, count, "out"), count, None))
 
 
 def _device_copy(source, target, count):
-    sa = _need(_span(source), count, "source")
-    ta = _need(_span(target), count, "target")
+    sa = _at(source, count, "source")
+    ta = _at(target, count, "target")
     _check(lib.mi_memcpy(ta, sa, 2 * count, 2))
 
 
 def _device_linear(x, weight, bias, out, rows, in_features, out_features):
-    xa = _need(_span(x), rows * in_features, "x")
-    wa = _need(_span(weight), out_features * in_features, "weight")
-    ba = _need(_span(bias), out_features, "bias") if bias is not None else None
-    oa = _need(_span(out), rows * out_features, "out")
+    xa = _at(x, rows * in_features, "x")
+    wa = _at(weight, out_features * in_features, "weight")
+    ba = _at(bias, out_features, "bias") if bias is not None else None
+    oa = _at(out, rows * out_features, "out")
     _check(lib.mi_linear(xa, wa, ba, oa, rows, in_features, out_features, None))
 
 
 def _device_linear_accumulate(x, weight, out: FloatTensor, rows, in_features, out_features):
     """out += x @ weight.T in fp32: a projection added into the residual
     stream with no fp16 rounding (bindings_device.cpp:351-365)."""
-    xa = _need(_span(x), rows * in_features, "x")
-    wa = _need(_span(weight), out_features * in_features, "weight")
+    xa = _at(x, rows * in_features, "x")
+    wa = _at(weight, out_features * in_features, "weight")
     oa = _floats(out, rows * out_features, "out")
     _check(lib.mi_linear_f32(xa, wa, oa, 1, rows, in_features, out_features, None))
 
 
 def _device_embed(ids: DeviceIndex, table, out, hidden, vocab):
-    ta = _need(_span(table), vocab * hidden, "table")
-    oa = _need(_span(out), ids.count * hidden, "out")
+    ta = _at(table, vocab * hidden, "table")
+    oa = _at(out, ids.count * hidden, "out")
     _check(lib.mi_embed(ids.address, ids.count, ta, oa, 0, hidden, vocab, None))
 
 
 def _device_embed_f32(ids: DeviceIndex, table, out: FloatTensor, hidden, vocab):
     """The embedding gather, widened exactly to fp32 (bindings_device.cpp:321-334)."""
-    ta = _need(_span(table), vocab * hidden, "table")
+    ta = _at(table, vocab * hidden, "table")
     oa = _floats(out, ids.count * hidden, "out")
     _check(lib.mi_embed(ids.address, ids.count, ta, oa, 1, hidden, vocab, None))
 
@@ -1402,8 +1423,8 @@ def scratch_elements(rows: int, vocab: int) -> int:
 def _logits_args(x, head, scratch, first_row, rows, hidden, vocab):
     _non_negative(first_row, "first_row")
     _non_negative(rows, "rows")
-    xa = _need(_span(x), (first_row + rows) * hidden, "x")
-    ha = _need(_span(head), vocab * hidden, "head")
+    xa = _at(x, (first_row + rows) * hidden, "x")
+    ha = _at(head, vocab * hidden, "head")
     sp = _span(scratch)
     sa = _need(sp, scratch_elements(rows, vocab), "scratch")
     return xa, ha, sa, sp.count
