@@ -76,18 +76,17 @@ namespace mi
     constexpr int kPageTokens = 32;
     constexpr int kMaxGroup = 16;
     constexpr int kMaxHeads = 64;
-    // Pages a split of one layer's launch takes, a wave each: half a
-    // workgroup's waves where the launch then still has no more workgroups
-    // than the device has CUs, so that a wave has a SIMD to itself (the rest
-    // of the workgroup idles); otherwise all of them. 28 layers at 4,999
-    // positions of the 1.5B shape with the key bias: 438 -> 382 us a token,
-    // at 15,000 (236 workgroups) 445 -> 400; at 32,768, where halving the
-    // pages would double the workgroups past the CUs, 403 -> 496.
-    __host__ __device__ inline int split_pages_of(int pages, int kv_heads, int cus)
+    // Pages a split of one layer's launch takes, a wave each, by the pages
+    // attended: up to `two` of them a quarter of a workgroup's waves, up to
+    // `four` half, otherwise all (the rest of the workgroup idles).
+    struct SplitRule
     {
-      return static_cast<long long>((pages + kWaves / 2 - 1) / (kWaves / 2)) * kv_heads <= cus
-                 ? kWaves / 2
-                 : kWaves;
+      int two;
+      int four;
+    };
+    __host__ __device__ inline int split_waves_of(const SplitRule &r, int pages)
+    {
+      return pages <= r.two ? 2 : pages <= r.four ? 4 : kWaves;
     }
 
     constexpr int kOwnPage = 0xFE; // the query's own page: open page + chunk rows
@@ -126,10 +125,6 @@ namespace mi
       int pages;
       int pages_per_wave;
       int splits;
-      // Waves of a split's workgroup that take pages (split_pages_of), and
-      // the device's CUs, by which a live launch chooses it.
-      int split_waves;
-      int cus;
       float scale; // 1/sqrt(hd) * log2 e: scores in base-2 units
       // Streaming launches: the (layer, KV-head block, page) units split into
       // stream_ranges equal contiguous ranges. A range is walked by
@@ -209,6 +204,10 @@ namespace mi
       std::uint16_t *row_normed;
       int row_hidden;
       float row_eps;
+      // Waves of a split's workgroup that take pages, and the rule by which a
+      // live launch chooses them.
+      int split_waves;
+      SplitRule split_rule;
     };
 
     __device__ inline half8 as_half8(u32x4 v) { return __builtin_bit_cast(half8, v); }
@@ -224,7 +223,7 @@ namespace mi
         a.seq_k = seq_k;
         a.start = seq_k - 1;
         a.live_pages = (seq_k + kPageTokens - 1) / kPageTokens;
-        a.split_waves = split_pages_of(a.live_pages, a.value_kv_heads, a.cus);
+        a.split_waves = split_waves_of(a.split_rule, a.live_pages);
         a.live_splits = (a.live_pages + a.split_waves - 1) / a.split_waves;
       }
     }
@@ -922,9 +921,9 @@ namespace mi
       const unsigned long long *table = a.table + layer * a.table_stride;
       const std::uint8_t *tiers = a.tiers != nullptr ? a.tiers + layer * a.table_stride : nullptr;
       const int own = a.causal ? (a.seq_k - 1) / kPageTokens : -1;
-      const int p0 = wave < a.split_waves
-                         ? (split * a.split_waves + wave) * a.pages_per_wave
-                         : a.live_pages; // an idle wave: no pages
+      // (An idle wave starts past the last page.)
+      const int p0 = (split * a.split_waves + wave) * a.pages_per_wave +
+                     (wave < a.split_waves ? 0 : a.live_pages);
       // The wave's pages: p0 and the next pages_per_wave - 1 (several a
       // wave), or p0 and every split_waves * busy pages on (the pages past the
       // busy splits).
@@ -2314,6 +2313,20 @@ namespace mi
       return stream_workspace(stream, floats);
     }
 
+    // Half the waves up to a workgroup a CU: a wave then has a SIMD to itself.
+    // 28 layers of the 1.5B shape at 15,000 positions with the key bias (236
+    // workgroups): 445 -> 400 us a token; at 32,768, where halving would make
+    // two workgroups a CU, 403 -> 496. A quarter up to five workgroups for
+    // eight CUs: a wave has half the CU's LDS traffic (the key bias's, above
+    // all) to itself, at 4,999 positions 384 -> 358, 267 -> 258 at
+    // 1,000 with no bias; past that the combine's
+    // further splits cost more.
+    SplitRule split_rule_of(int kv_heads)
+    {
+      const int cus = device_multiprocessors();
+      return {cus * 5 / 8 / kv_heads * 2, cus / kv_heads * 4};
+    }
+
     bool aligned16(const void *p) { return (reinterpret_cast<std::uintptr_t>(p) & 15u) == 0; }
 
     // Waves of the head_dim-64 pages kernel (a wave a page of one KV head)
@@ -2490,7 +2503,7 @@ namespace mi
     d.value_kv_heads = a.kv_heads;
     d.stat_group = group;
     d.pages = pages;
-    d.cus = device_multiprocessors();
+    d.split_rule = split_rule_of(a.kv_heads);
     d.split_waves = kWaves;
     // Scores in base-2 units: the softmax weights are exp2 of them.
     d.scale = static_cast<float>(1.4426950408889634 / std::sqrt(static_cast<double>(a.head_dim)));
@@ -2573,12 +2586,14 @@ namespace mi
     }
     else if (ls.split)
     {
-      // (A live launch may see fewer pages: `splits` holds the most any
-      // count up to `pages` makes, in every launch, so that kept statistics
-      // have one layout.)
+      // `splits` is this launch's, or, where it may see fewer pages (a live
+      // one) or its statistics are kept for a fold that may, the most that
+      // any count up to `pages` makes.
       d.pages_per_wave = 1;
-      d.splits = decode_splits(a.kv_heads, pages);
-      d.split_waves = split_pages_of(pages, a.kv_heads, d.cus);
+      d.split_waves = split_waves_of(d.split_rule, pages);
+      d.splits = ls.live_seq_k != nullptr || ls.keep_ml != nullptr
+                     ? decode_splits(a.kv_heads, pages)
+                     : (pages + d.split_waves - 1) / d.split_waves;
     }
     else
     {
@@ -2733,10 +2748,9 @@ namespace mi
 
   int decode_splits(int kv_heads, int pages)
   {
-    constexpr int kHalf = kWaves / 2;
-    const int most_halved = device_multiprocessors() / kv_heads; // workgroups a KV head
-    return std::max((pages + kWaves - 1) / kWaves,
-                    std::min((pages + kHalf - 1) / kHalf, most_halved));
+    const SplitRule r = split_rule_of(kv_heads);
+    return std::max({(pages + kWaves - 1) / kWaves, (std::min(pages, r.four) + 3) / 4,
+                     (std::min(pages, r.two) + 1) / 2});
   }
 
   std::size_t decode_kept_floats(int heads, int kv_heads, int seq_k)
@@ -2762,8 +2776,8 @@ namespace mi
     d.pages = pages;
     d.seq_k = f.seq_k;
     d.splits = decode_splits(f.kv_heads, pages);
-    d.cus = device_multiprocessors();
-    d.split_waves = split_pages_of(pages, f.kv_heads, d.cus);
+    d.split_rule = split_rule_of(f.kv_heads);
+    d.split_waves = split_waves_of(d.split_rule, pages);
     d.split_ml = f.kept;
     d.page_stats = f.kept + static_cast<std::size_t>(f.layers) * f.heads * d.splits * 2;
     d.mass = f.mass;

@@ -1,5 +1,5 @@
-"""One layer's decode where its split changes: half a workgroup's waves a
-split up to a workgroup a CU, all of them past it. Outputs and masses against
+"""One layer's decode where its split changes: a quarter of a workgroup's
+waves a split, half of them up to a workgroup a CU, all of them past it. Outputs and masses against
 the float64 oracle on both sides; a launch sized for a long context with its
 seq_k on the device, and the statistics kept for a later fold, to the bits of
 the plain launch at every seq_k."""
@@ -35,7 +35,9 @@ def cache_of(seq, kv, hd, most):
 def test_decode_on_both_sides_of_the_split(heads, kv, hd, bias):
     m = mi()
     d = m.device
-    # The pages at which halved splits would pass a workgroup a CU (256 CUs).
+    # The pages past which splits of two would make more than five workgroups
+    # for eight CUs, and of four more than one a CU (256 CUs).
+    two = 160 // kv * 2 * P
     edge = 256 // kv * 4 * P
     most = edge + 3 * P
     rng = np.random.default_rng(heads + hd + bias)
@@ -47,7 +49,7 @@ def test_decode_on_both_sides_of_the_split(heads, kv, hd, bias):
         rope.cover(most)
     part = d.empty_f32(d.attention_partials(hd))
     q = [put(normal(rng, heads, hd)) for _ in range(LAYERS)]
-    for seq in (1, P + 1, 5 * P, edge, edge + 1, edge + 2 * P + 7):
+    for seq in (1, P + 1, 5 * P, two, two + 1, edge, edge + 1, edge + 2 * P + 7):
         alloc, cache = cache_of(seq, kv, hd, most)
         for l in range(LAYERS):
             if seq > 1:
