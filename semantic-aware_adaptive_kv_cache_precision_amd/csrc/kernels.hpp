@@ -5,6 +5,8 @@
 
 #include "common.hpp"
 
+#include <mutex>
+
 namespace mi
 {
 
@@ -323,8 +325,12 @@ namespace mi
   // where none can be had (the launch then takes the path that needs none).
   // `growing_to`: the bytes the same queries would need once the owner is
   // full, so that a prompt's chunks do not outgrow it one after the other.
+  // A chunk is several launches that hand data to each other there, so the
+  // caller holds order() from the request to its last launch: another
+  // thread's chunk on the same stream then follows it whole.
   struct StreamScratch
   {
+    virtual std::unique_lock<std::mutex> order() = 0;
     virtual void *take(hipStream_t stream, std::size_t bytes, std::size_t growing_to) = 0;
 
   protected:

@@ -110,6 +110,10 @@ namespace mi
   void *StreamBuffers::take(hipStream_t stream, std::size_t bytes, std::size_t growing_to)
   {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (stream == hipStreamPerThread)
+    {
+      return nullptr;
+    }
     if (hipStreamIsCapturing(stream, &capturing) != hipSuccess)
     {
       (void)hipGetLastError();
@@ -119,7 +123,6 @@ namespace mi
     {
       return nullptr;
     }
-    std::lock_guard<std::mutex> hold(lock_);
     auto at = std::find_if(held_.begin(), held_.end(),
                            [&](const auto &entry) { return entry.first == stream; });
     if (at == held_.end())

@@ -136,19 +136,24 @@ namespace mi
 
   // A buffer a stream, of one owner's, for launches that hand data to each
   // other on that stream alone. Bounded: kMost streams (a buffer each, as
-  // large as its largest request); a further stream gets none, nor does a
+  // large as its largest request); a further stream gets none, nor do the
+  // per-thread default streams, one handle for many streams, nor does a
   // stream that is being captured, whose graph could be replayed beside
   // other work of the owner's, nor a request the device has no memory for.
   // Grown buffers and the owner's end give the old ones back, once the
-  // device is idle. Safe with several threads.
+  // device is idle. take() is called with order() held.
   class StreamBuffers final : public StreamScratch
   {
   public:
+    std::unique_lock<std::mutex> order() override
+    {
+      return std::unique_lock<std::mutex>(order_);
+    }
     void *take(hipStream_t stream, std::size_t bytes, std::size_t growing_to) override;
 
   private:
     static constexpr std::size_t kMost = 4;
-    std::mutex lock_;
+    std::mutex order_;
     std::vector<std::pair<hipStream_t, std::unique_ptr<DeviceBuffer>>> held_;
   };
 

@@ -2,6 +2,9 @@
 its tiles, steps, splits and dispatch end, against the float64 oracle at the
 attention gate (conftest.ATTN_MAX_REL, with the oracle's fp32 error bound)."""
 
+import threading
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -106,3 +109,43 @@ def test_captures_and_further_streams_take_the_staging_path():
             m.set_stream(None)
         s.synchronize()
         assert_attention_close(out.to_numpy().reshape(q.shape), want, f"stream {i}", bound)
+
+
+def test_two_threads_chunks_on_one_stream_keep_their_own_layout():
+    """Chunks of two layers from two threads, both on the null stream: the
+    scratch is the stream's, so each chunk's launches follow the other's
+    whole. Every output has the bits of the call by itself."""
+    m = mi()
+    d = m.device
+    heads, kv, hd, seq, seq_q, calls = 32, 8, 64, P * 40 + 4, 64, 24
+    rng = np.random.default_rng(5)
+    alloc, cache = pages_for(P, kv, hd, 0)
+    for layer in (0, 1):
+        store_in_runs(cache, layer, normal(rng, seq, kv, hd), normal(rng, seq, kv, hd), [seq])
+    dq = put(normal(rng, seq_q, heads, hd))
+    n = seq_q * heads * hd
+
+    def attend(layer, out):
+        cache.attention(layer, dq, None, None, out, seq_q, seq, heads, kv, hd, None, None, None,
+                        None)
+
+    want = []
+    for layer in (0, 1):
+        out = d.empty(n)
+        attend(layer, out)
+        want.append(out.to_numpy())
+    outs = [[d.empty(n) for _ in range(calls)] for _ in (0, 1)]
+    start = threading.Barrier(2)
+
+    def work(layer):
+        start.wait()
+        for out in outs[layer]:
+            attend(layer, out)
+
+    announce("chunks from two threads")
+    with ThreadPoolExecutor(2) as pool:
+        list(pool.map(work, (0, 1)))
+    m.synchronize()
+    for layer in (0, 1):
+        for i, out in enumerate(outs[layer]):
+            assert np.array_equal(out.to_numpy(), want[layer]), (layer, i)
