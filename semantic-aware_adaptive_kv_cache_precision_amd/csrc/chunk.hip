@@ -801,7 +801,7 @@ namespace mi
 
   bool chunk_applies(const KVSource &kv, const AttentionArgs &a)
   {
-    return a.seq_q >= kChunkQueries && kv.layout != Layout::kContiguous &&
+    return a.seq_q >= kChunkQueries * (a.head_dim == 64 ? 2 : 1) && kv.layout != Layout::kContiguous &&
            a.heads / a.kv_heads <= block_rows(1) && prefill_applies(kv, a);
   }
 

@@ -17,13 +17,13 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("heads,kv,hd,seq,seq_q,bias", [
-    (32, 8, 64, P * 5 + 3, 63, False),     # the largest chunk that stages page by page
-    (32, 8, 64, P * 5 + 3, 64, False),     # the smallest over laid-out pages
-    (32, 8, 64, 64, 64, False),            # a prompt of whole pages, nothing before it
-    (32, 8, 64, P * 7 + 31, 65, True),     # one query past a workgroup's 64
+    (32, 8, 64, P * 5 + 3, 127, False),     # the largest chunk that stages page by page
+    (32, 8, 64, P * 5 + 3, 128, False),     # the smallest over laid-out pages
+    (32, 8, 64, 128, 128, False),            # a prompt of whole pages, nothing before it
+    (32, 8, 64, P * 7 + 31, 129, True),     # one query past two workgroups' 64
     (4, 4, 64, P * 9 + 1, 257, False),     # a head a KV head: 256 queries a workgroup, and one
-    (16, 1, 64, P * 6, 90, False),         # sixteen heads a KV head
-    (14, 2, 64, P * 33 + 17, 73, True),    # rows that do not fill their tiles; steps in splits
+    (16, 1, 64, P * 6, 154, False),         # sixteen heads a KV head
+    (14, 2, 64, P * 33 + 17, 137, True),    # rows that do not fill their tiles; steps in splits
     (12, 2, 128, P * 3 + 2, 64, True),     # head_dim 128: 21 queries a workgroup
     (12, 2, 128, P * 40 + 30, 150, False),
     (12, 2, 128, P * 130 + 5, 64, True),   # many splits of few queries
@@ -47,7 +47,7 @@ def test_one_score_far_above_the_rest_moves_the_reference(heads, kv, hd):
     next, and fall again: each row's softmax reference moves up step by step
     and its earlier sums vanish."""
     rng = np.random.default_rng(2)
-    seq, seq_q = P * 12 + 5, 70
+    seq, seq_q = P * 12 + 5, 134
     k, v = normal(rng, seq, kv, hd), normal(rng, seq, kv, hd)
     q = normal(rng, seq_q, heads, hd)
     for page, size in ((1, 4.0), (3, 12.0), (4, 40.0), (8, 6.0)):
@@ -70,7 +70,7 @@ def test_captures_and_further_streams_take_the_staging_path():
     program's own calls."""
     m = mi()
     d = m.device
-    heads, kv, hd, seq, seq_q = 32, 8, 64, P * 9 + 4, 80
+    heads, kv, hd, seq, seq_q = 32, 8, 64, P * 9 + 4, 144
     rng = np.random.default_rng(9)
     k, v, q = (normal(rng, seq, kv, hd), normal(rng, seq, kv, hd), normal(rng, seq_q, heads, hd))
     alloc, cache = pages_for(P, kv, hd, 0)
@@ -117,7 +117,7 @@ def test_two_threads_chunks_on_one_stream_keep_their_own_layout():
     whole. Every output has the bits of the call by itself."""
     m = mi()
     d = m.device
-    heads, kv, hd, seq, seq_q, calls = 32, 8, 64, P * 40 + 4, 64, 24
+    heads, kv, hd, seq, seq_q, calls = 32, 8, 64, P * 40 + 4, 128, 24
     rng = np.random.default_rng(5)
     alloc, cache = pages_for(P, kv, hd, 0)
     for layer in (0, 1):
