@@ -34,7 +34,7 @@
 //
 // Precision as in prefill.hip: Q and the dequantised K and V exact in fp16,
 // k + bias as fp16 high and low parts of the fp32 sum, the probabilities as
-// high and low parts of p * 2^5 (kProbScale2), sums in fp32.
+// high and low parts of p * 2^14 (kProbScale2), sums in fp32.
 //
 // Causality: rows read each page before their own sealed and their own at
 // FP16 (both versions of the chunk's own pages are laid out). A step no row
@@ -60,15 +60,20 @@ namespace mi
     constexpr int kChunkWaves = 4;
     constexpr int kChunkThreads = 64 * kChunkWaves;
     constexpr int kTileRows = 32; // rows a product takes
-    // A row's probabilities are held x 2^5 against its reference, the maximum
-    // of some earlier step: a step whose probabilities stay within fp16 (their
-    // sum, no less than any of them, at most kMostSum) leaves it, so that the
-    // maximum of most steps is never formed, and a row's maximum may rise by
-    // 10 powers of two before it moves. The low part's last bit is 2^-30 of
-    // the reference's weight, below an fp32 sum's.
-    constexpr float kProbScale2 = 5.0f;
-    constexpr float kProbUnscale = 1.0f / 32.0f;
-    constexpr float kMostSum = 46000.0f;
+    // A row's probabilities are held x 2^14 against its reference, which is
+    // never above the row's maximum so far: the low part's last bit is then at
+    // most 2^-38 of the largest probability's weight, as where the reference
+    // is the maximum itself (prefill.hip). A step whose probabilities stay
+    // within fp16 (a part of their sum, no less than any in it, shows it)
+    // leaves the reference, so that the maximum of most steps is never formed
+    // and a row's maximum may rise by two powers of two before it moves: a
+    // wave's rows then move it in a sixth of its steps. (A 2,048-query chunk
+    // at 16K: 416 us; 420 with every step's maximum formed; 386 with the
+    // probabilities held x 2^5, which leaves the maximum ten powers to rise
+    // but the low part nine bits fewer.)
+    constexpr float kProbScale2 = 14.0f;
+    constexpr float kProbUnscale = 1.0f / 16384.0f;
+    constexpr float kMostProb = 65504.0f; // fp16's largest value
     constexpr int kMaxSplits = 32;
 
     struct ChunkArgs
@@ -330,11 +335,12 @@ namespace mi
     }
 
     // Scores of N pages to probabilities (x 2^kProbScale2) in place; returns
-    // the lane's sum of them.
+    // the lane's sum of them, and in `most` the largest of its four parts, no
+    // less than any probability.
     template <int N>
-    __device__ inline float exponentiate(f32x16 (&s)[N], float scale2, float shift2)
+    __device__ inline float exponentiate(f32x16 (&s)[N], float scale2, float shift2, float &most)
     {
-      float sum[2] = {0.0f, 0.0f};
+      float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int j = 0; j < N; ++j)
       {
@@ -342,10 +348,52 @@ namespace mi
         for (int i = 0; i < 16; ++i)
         {
           s[j][i] = __builtin_amdgcn_exp2f(fmaf(s[j][i], scale2, shift2));
-          sum[i % 2] += s[j][i];
+          part[i % 4] += s[j][i];
         }
       }
-      return sum[0] + sum[1];
+      most = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+      return (part[0] + part[1]) + (part[2] + part[3]);
+    }
+
+    // Probabilities of N pages (finite) brought back within fp16, with their
+    // sum and the row's sum and outputs, by the power of two that puts the
+    // row's largest, where it is larger, in [2^14, 2^15): nothing is rounded.
+    template <int HD, int N>
+    __device__ inline void lower(f32x16 (&p)[N], float &sum, Rows<HD> &run)
+    {
+      float top = 0.0f;
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+      {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+        {
+          top = fmaxf(top, p[j][i]);
+        }
+      }
+      const int by = max(__builtin_amdgcn_frexp_expf(lane_max32(top)) - 15, 0);
+      const float factor = __builtin_ldexpf(1.0f, -by);
+      run.m += static_cast<float>(by);
+      run.l *= factor;
+      sum *= factor;
+#pragma unroll
+      for (int dt = 0; dt < HD / 32; ++dt)
+      {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+        {
+          run.o[dt][i] *= factor;
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+      {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+        {
+          p[j][i] *= factor;
+        }
+      }
     }
 
     // P.V of a page added, each operand read for every row tile, the outputs'
@@ -513,33 +561,49 @@ namespace mi
         return stages + buf * kStage;
       };
       int step = begin;
-      for (; step < min(end, whole_steps); ++step)
+      const std::uint16_t *stage = begin < end ? turn(begin) : stages;
+      const int whole_end = min(end, whole_steps);
+      // The rows' first reference: their maximum over the first page, which
+      // every row reads.
+      if (step < whole_end)
       {
-        const std::uint16_t *stage = turn(step);
-        f32x16 s[RT][NP];
-        // A wave in its products goes before one in its softmax, so that the
-        // two workgroups of a CU alternate (a 2,048-query chunk at 16K: 398
-        // to 382 us).
-        __builtin_amdgcn_s_setprio(1);
-        page_scores<HD, RT, NP, kBias>(s, stage, qf, lane);
-        __builtin_amdgcn_s_setprio(0);
-        // (A row with no reference yet: the sum is infinite or no number.)
-        float sum[RT];
-        bool past = false;
+        f32x16 s[RT][1];
+        page_scores<HD, RT, 1, kBias>(s, stage, qf, lane);
 #pragma unroll
         for (int t = 0; t < RT; ++t)
         {
-          sum[t] = exponentiate<NP>(s[t], a.scale2, kProbScale2 - run[t].m);
-          past = past || !(sum[t] <= kMostSum);
+          move_reference<HD, 1>(s[t], a.scale2, run[t]);
         }
-        if (__any(past))
-        {
-          page_scores<HD, RT, NP, kBias>(s, stage, qf, lane);
+      }
+      while (step < whole_end)
+      {
+        f32x16 s[RT][NP];
+        // A wave in its products goes before one in its softmax, so that the
+        // two workgroups of a CU alternate (a 2,048-query chunk at 16K, the
+        // probabilities x 2^5: 398 to 382 us).
+        __builtin_amdgcn_s_setprio(1);
+        page_scores<HD, RT, NP, kBias>(s, stage, qf, lane);
+        __builtin_amdgcn_s_setprio(0);
+        float sum[RT], most[RT];
+        bool finite = true;
 #pragma unroll
-          for (int t = 0; t < RT; ++t)
+        for (int t = 0; t < RT; ++t)
+        {
+          sum[t] = exponentiate<NP>(s[t], a.scale2, kProbScale2 - run[t].m, most[t]);
+          finite = finite && sum[t] < INFINITY;
+        }
+        // A rise past fp32's range, a row whose first page had no finite score,
+        // or values that are not finite: the wave goes on below.
+        if (!__all(finite))
+        {
+          break;
+        }
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+        {
+          if (__any(most[t] > kMostProb))
           {
-            move_reference<HD, NP>(s[t], a.scale2, run[t]);
-            sum[t] = exponentiate<NP>(s[t], a.scale2, shift_of(run[t].m));
+            lower<HD, NP>(s[t], sum[t], run[t]);
           }
         }
 #pragma unroll
@@ -554,12 +618,16 @@ namespace mi
           page_values<HD, RT, NP>(stage + j * kBlock + kV, s, j, run, lane);
         }
         __builtin_amdgcn_s_setprio(0);
+        if (++step < end)
+        {
+          stage = turn(step);
+        }
       }
-      // The rest page by page: a page no row of the wave reads is left out,
-      // whatever it holds; a masked key's score is -inf.
-      for (; step < end; ++step)
+      // The rest page by page, against the exact maximum: a page no row of
+      // the wave reads is left out, whatever it holds; a masked key's score
+      // is -inf.
+      while (step < end)
       {
-        const std::uint16_t *stage = turn(step);
         const bool sealed = step < sealed_steps;
         const int p0 = sealed ? NP * step : own_from + NP * (step - sealed_steps);
         for (int j = 0; j < NP; ++j)
@@ -587,9 +655,14 @@ namespace mi
               s[t][0][i] = key <= limit ? s[t][0][i] : -INFINITY;
             }
             move_reference<HD, 1>(s[t], a.scale2, run[t]);
-            run[t].l += exponentiate<1>(s[t], a.scale2, shift_of(run[t].m));
+            float most;
+            run[t].l += exponentiate<1>(s[t], a.scale2, shift_of(run[t].m), most);
           }
           page_values<HD, RT, 1>(stage + j * kBlock + kV, s, 0, run, lane);
+        }
+        if (++step < end)
+        {
+          stage = turn(step);
         }
       }
 

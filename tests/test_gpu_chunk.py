@@ -64,6 +64,34 @@ def test_one_score_far_above_the_rest_moves_the_reference(heads, kv, hd):
                            att.attention_bound(q, k, v, w))
 
 
+@pytest.mark.parametrize("heads,kv,hd,seq_q,high", [(32, 8, 64, 134, 2.162109375),
+                                                       (12, 2, 128, 160, 1.509765625)])
+def test_small_probabilities_keep_their_bits(heads, kv, hd, seq_q, high):
+    """One key far above 8,191 others whose values are all the output: each of
+    theirs is some 2^-25 of its weight, of which fp16 high and low parts of
+    p x 2^14 hold 2^-14 at least (their last bit is 2^-38 of the weight; of
+    p x 2^5 it would be 2^-29, a thirtieth of such a probability). Besides it
+    the outputs part from float64 by the fp16 store's rounding and fp32
+    exponents and sums (2^-16)."""
+    seq = P * 256
+    m = mi()
+    d = m.device
+    k, v = np.zeros((seq, kv, hd), np.float32), np.full((seq, kv, hd), 4096.0, np.float32)
+    k[0], v[0] = high, 0.0
+    q = np.ones((seq_q, heads, hd), np.float32)
+    alloc, cache = pages_for(P, kv, hd, 0)
+    store_in_runs(cache, 0, k, v, [seq])
+    out = d.empty(q.size)
+    announce("chunk small probabilities", heads, kv, hd)
+    cache.attention(0, put(q), None, None, out, seq_q, seq, heads, kv, hd, None, None, None, None)
+    keys = np.arange(seq - seq_q, seq)  # keys besides the first that a query reads
+    weight = keys * np.exp(-high * np.sqrt(float(hd)))
+    want = 4096.0 * weight / (1.0 + weight)
+    got = out.to_numpy().reshape(seq_q, -1)
+    error = np.abs(got / want[:, None] - 1.0).max()
+    assert error < 2.0**-11 + 2.0**-14 + 2.0**-16, error
+
+
 def test_captures_and_further_streams_take_the_staging_path():
     """A captured launch and a fifth stream get no scratch and take the path
     that needs none: the same attention, the graph replayed between the
