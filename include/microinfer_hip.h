@@ -518,6 +518,13 @@ typedef struct mi_kv_info {
   size_t page_bytes, kv_width, shadow_count, shadow_bytes;
 } mi_kv_info;
 int mi_kv_info_get(mi_kv_pages *kv, mi_kv_info *out);
+/* The scratch a long chunk's attention lays its pages out in (no counterpart
+ * in the reference): how many chunks the cache has laid out so, and the bytes
+ * it holds now. The cache keeps it for its next chunk; mi_release_chunk_scratch
+ * gives every cache's back (waiting for the chunks that use it), as an
+ * allocation of this library does by itself when the device is out of memory. */
+int mi_kv_chunk_scratch(mi_kv_pages *kv, size_t *chunks, size_t *bytes);
+int mi_release_chunk_scratch(size_t *bytes);
 int mi_kv_birth_tier(mi_kv_pages *kv, int layer, int page, int *tier);
 /* last_move: has, layer, page, from, to; bytes; seconds. */
 int mi_kv_last_move(mi_kv_pages *kv, int *has, int *ints4, size_t *bytes2, double *seconds2);

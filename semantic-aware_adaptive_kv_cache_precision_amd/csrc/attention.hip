@@ -483,11 +483,11 @@ namespace mi
       AttentionArgs full = a;
       full.seq_k = std::max(a.seq_k, a.capacity);
       const auto order = a.chunk_scratch->order();
-      void *scratch = a.chunk_scratch->take(stream, chunk_workspace_bytes(kv, a),
-                                            chunk_workspace_bytes(kv, full));
-      if (scratch != nullptr)
+      const ChunkScratch::Taken scratch = a.chunk_scratch->take(
+          stream, chunk_workspace_bytes(kv, a), chunk_workspace_bytes(kv, full));
+      if (scratch.bytes != nullptr)
       {
-        launch_chunk(kv, a, scratch, stream);
+        launch_chunk(kv, a, scratch.bytes, scratch.done, stream);
         return;
       }
     }

@@ -330,7 +330,7 @@ int mi_malloc(void **out, size_t bytes)
     *out = nullptr;
     if (bytes > 0)
     {
-      mi::hip_check(hipMalloc(out, bytes), "hipMalloc");
+      *out = mi::device_alloc(bytes);
     }
   });
 }
@@ -1591,6 +1591,19 @@ int mi_kv_info_get(mi_kv_pages *kv, mi_kv_info *out)
     out->shadow_count = k.shadows().count();
     out->shadow_bytes = k.shadows().bytes();
   });
+}
+
+int mi_kv_chunk_scratch(mi_kv_pages *kv, size_t *chunks, size_t *bytes)
+{
+  return guarded([&] {
+    *chunks = kv->impl.chunk_scratch().taken();
+    *bytes = kv->impl.chunk_scratch().bytes();
+  });
+}
+
+int mi_release_chunk_scratch(size_t *bytes)
+{
+  return guarded([&] { *bytes = mi::release_chunk_scratch(); });
 }
 
 int mi_kv_birth_tier(mi_kv_pages *kv, int layer, int page, int *tier)

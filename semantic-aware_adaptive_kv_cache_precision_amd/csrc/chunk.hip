@@ -44,6 +44,8 @@
 #include "chunk_pages.hpp"
 #include "lane_ops.hpp"
 
+#include <hip/hip_ext.h>
+
 #include <algorithm>
 #include <cmath>
 
@@ -764,7 +766,7 @@ namespace mi
 
     // The launches, or with a null workspace only the bytes it needs.
     template <int HD, int RT, int NP, bool kBias, int kWavesASimd>
-    std::size_t run(ChunkArgs args, std::uint8_t *work, hipStream_t stream)
+    std::size_t run(ChunkArgs args, std::uint8_t *work, hipEvent_t done, hipStream_t stream)
     {
       args.qb = std::min(args.seq_q, block_rows(RT) / args.group);
       auto kernel = chunk_kernel<HD, RT, NP, kBias, kWavesASimd>;
@@ -825,22 +827,25 @@ namespace mi
       hipLaunchKernelGGL((lay_out_kernel<HD, kBias>), dim3(written, args.kv_heads), dim3(256), 0,
                          stream, args);
       hip_check(hipGetLastError(), "chunk layout kernel launch");
-      hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks * args.splits)),
-                         dim3(kChunkThreads), kLds, stream, args);
+      // The last launch signals `done` with its own completion: no packet of
+      // its own on the stream (an event recorded after it takes 1 to 3 us).
+      hipExtLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks * args.splits)),
+                            dim3(kChunkThreads), kLds, stream, nullptr,
+                            args.splits > 1 ? nullptr : done, 0, args);
       hip_check(hipGetLastError(), "chunk kernel launch");
       if (args.splits > 1)
       {
         const std::size_t threads = rows * (HD / 4);
-        hipLaunchKernelGGL(chunk_combine_kernel<HD>,
-                           dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream,
-                           args, rows);
+        hipExtLaunchKernelGGL(chunk_combine_kernel<HD>,
+                              dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0,
+                              stream, nullptr, done, 0, args, rows);
         hip_check(hipGetLastError(), "chunk combine kernel launch");
       }
       return needed;
     }
 
     std::size_t dispatch(const KVSource &kv, const AttentionArgs &a, std::uint8_t *work,
-                         hipStream_t stream)
+                         hipEvent_t done, hipStream_t stream)
     {
       ChunkArgs args{};
       args.kv = kv;
@@ -863,11 +868,11 @@ namespace mi
       args.scale2 = 1.4426950408889634f / std::sqrt(static_cast<float>(a.head_dim));
       if (a.head_dim == 128)
       {
-        return a.k_bias != nullptr ? run<128, 1, 1, true, 2>(args, work, stream)
-                                   : run<128, 1, 2, false, 2>(args, work, stream);
+        return a.k_bias != nullptr ? run<128, 1, 1, true, 2>(args, work, done, stream)
+                                   : run<128, 1, 2, false, 2>(args, work, done, stream);
       }
-      return a.k_bias != nullptr ? run<64, 2, 2, true, 2>(args, work, stream)
-                                 : run<64, 2, 2, false, 2>(args, work, stream);
+      return a.k_bias != nullptr ? run<64, 2, 2, true, 2>(args, work, done, stream)
+                                 : run<64, 2, 2, false, 2>(args, work, done, stream);
     }
 
   } // namespace
@@ -880,13 +885,13 @@ namespace mi
 
   std::size_t chunk_workspace_bytes(const KVSource &kv, const AttentionArgs &a)
   {
-    return dispatch(kv, a, nullptr, nullptr);
+    return dispatch(kv, a, nullptr, nullptr, nullptr);
   }
 
-  void launch_chunk(const KVSource &kv, const AttentionArgs &a, void *workspace,
+  void launch_chunk(const KVSource &kv, const AttentionArgs &a, void *workspace, hipEvent_t done,
                     hipStream_t stream)
   {
-    dispatch(kv, a, static_cast<std::uint8_t *>(workspace), stream);
+    dispatch(kv, a, static_cast<std::uint8_t *>(workspace), done, stream);
   }
 
 } // namespace mi

@@ -320,21 +320,26 @@ namespace mi
   // share one; launches on one stream are ordered by it.
   float *stream_workspace(hipStream_t stream, std::size_t count);
 
-  // Scratch of a chunk's attention (chunk.hip): at least `bytes` that are the
-  // launches' on `stream` until the next request for that stream, or null
-  // where none can be had (the launch then takes the path that needs none).
-  // `growing_to`: the bytes the same queries would need once the owner is
-  // full, so that a prompt's chunks do not outgrow it one after the other.
-  // A chunk is several launches that hand data to each other there, so the
-  // caller holds order() from the request to its last launch: another
-  // thread's chunk on the same stream then follows it whole.
-  struct StreamScratch
+  // Scratch of a chunk's attention (chunk.hip), one buffer for every stream.
+  // A chunk is several launches that hand data to each other there: the
+  // caller holds order() from the request to its last launch, so that another
+  // thread's chunk follows it whole, and its last launch signals the event
+  // that take() gives, which the next chunk's stream waits for.
+  struct ChunkScratch
   {
+    struct Taken
+    {
+      void *bytes;     // null where none can be had: the launch takes the path that needs none
+      hipEvent_t done; // for the last launch that uses them to signal
+    };
     virtual std::unique_lock<std::mutex> order() = 0;
-    virtual void *take(hipStream_t stream, std::size_t bytes, std::size_t growing_to) = 0;
+    // At least `bytes`. `growing_to`: what the same queries would need once
+    // the owner is full, so that a prompt's chunks do not outgrow the buffer
+    // one after the other.
+    virtual Taken take(hipStream_t stream, std::size_t bytes, std::size_t growing_to) = 0;
 
   protected:
-    ~StreamScratch() = default;
+    ~ChunkScratch() = default;
   };
 
   struct AttentionArgs
@@ -359,7 +364,7 @@ namespace mi
     float *partials;          // attention_partials_floats(hd) or null: no split
     std::size_t partials_floats; // its size, when the caller knows it (0: unknown)
     WorkspaceSource *workspace;  // the decode path's scratch, or null (see above)
-    StreamScratch *chunk_scratch; // a chunk's laid-out pages go here, or null: none
+    ChunkScratch *chunk_scratch; // a chunk's laid-out pages go here, or null: none
     int capacity;                // the positions the owner has room for; with chunk_scratch
   };
 
@@ -390,11 +395,11 @@ namespace mi
   // at 14/2 heads of 64, and after 32 positions 14.7 against 18.6, 12.1
   // against 11.3 and (32/8 of 64) 12.4 against 10.5.
   // `workspace` holds chunk_workspace_bytes and belongs to the launch until
-  // the stream is past it.
+  // `done`, which its last kernel signals.
   constexpr int kChunkQueries = 64;
   bool chunk_applies(const KVSource &kv, const AttentionArgs &a);
   std::size_t chunk_workspace_bytes(const KVSource &kv, const AttentionArgs &a);
-  void launch_chunk(const KVSource &kv, const AttentionArgs &a, void *workspace,
+  void launch_chunk(const KVSource &kv, const AttentionArgs &a, void *workspace, hipEvent_t done,
                     hipStream_t stream);
 
   // The decode fast path (decode.hip) over `layers` consecutive layers of one

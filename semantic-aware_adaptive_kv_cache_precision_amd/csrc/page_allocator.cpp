@@ -93,7 +93,7 @@ namespace mi
   {
     if (bytes > 0)
     {
-      hip_check(hipMalloc(&ptr_, bytes), "hipMalloc");
+      ptr_ = device_alloc(bytes);
     }
   }
 
@@ -107,48 +107,151 @@ namespace mi
     }
   }
 
-  void *StreamBuffers::take(hipStream_t stream, std::size_t bytes, std::size_t growing_to)
+  void *device_alloc(std::size_t bytes)
+  {
+    void *at = nullptr;
+    hipError_t made = hipMalloc(&at, bytes);
+    if (made == hipErrorOutOfMemory || made == hipErrorMemoryAllocation)
+    {
+      (void)hipGetLastError();
+      if (release_chunk_scratch() > 0)
+      {
+        made = hipMalloc(&at, bytes);
+      }
+    }
+    hip_check(made, "hipMalloc");
+    return at;
+  }
+
+  // ---- a chunk's scratch -----------------------------------------------------------------
+
+  namespace
+  {
+    // Every owner's scratch; never destroyed, as owners may go last.
+    struct ScratchList
+    {
+      std::mutex lock;
+      std::vector<OwnedChunkScratch *> all;
+    };
+    ScratchList &scratch_list()
+    {
+      static ScratchList &list = *new ScratchList;
+      return list;
+    }
+
+    // Allocations, frees and waits that a stream this thread captures neither
+    // records nor forbids.
+    class RelaxedCapture
+    {
+    public:
+      RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+      ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+
+    private:
+      hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+    };
+  } // namespace
+
+  OwnedChunkScratch::OwnedChunkScratch()
+  {
+    ScratchList &list = scratch_list();
+    std::lock_guard<std::mutex> hold(list.lock);
+    list.all.push_back(this);
+  }
+
+  OwnedChunkScratch::~OwnedChunkScratch()
+  {
+    {
+      ScratchList &list = scratch_list();
+      std::lock_guard<std::mutex> hold(list.lock);
+      list.all.erase(std::find(list.all.begin(), list.all.end(), this));
+    }
+    const RelaxedCapture relaxed;
+    drop();
+    if (done_ != nullptr)
+    {
+      (void)hipEventDestroy(done_);
+    }
+  }
+
+  void OwnedChunkScratch::drop()
+  {
+    if (buffer_ != nullptr)
+    {
+      (void)hipEventSynchronize(done_);
+      (void)hipFree(buffer_);
+      buffer_ = nullptr;
+      size_ = 0;
+    }
+  }
+
+  std::size_t OwnedChunkScratch::release()
+  {
+    const std::unique_lock<std::mutex> held(order_, std::try_to_lock);
+    if (!held.owns_lock())
+    {
+      return 0;
+    }
+    const RelaxedCapture relaxed;
+    const std::size_t bytes = size_;
+    drop();
+    return bytes;
+  }
+
+  ChunkScratch::Taken OwnedChunkScratch::take(hipStream_t stream, std::size_t bytes,
+                                              std::size_t growing_to)
   {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (stream == hipStreamPerThread)
-    {
-      return nullptr;
-    }
     if (hipStreamIsCapturing(stream, &capturing) != hipSuccess)
     {
       (void)hipGetLastError();
-      return nullptr;
+      return {nullptr, nullptr};
     }
     if (capturing != hipStreamCaptureStatusNone)
     {
-      return nullptr;
+      return {nullptr, nullptr};
     }
-    auto at = std::find_if(held_.begin(), held_.end(),
-                           [&](const auto &entry) { return entry.first == stream; });
-    if (at == held_.end())
+    if (size_ < bytes)
     {
-      if (held_.size() == kMost)
+      const RelaxedCapture relaxed;
+      // (The event orders kernels on one device: no fence to the host.)
+      if (done_ == nullptr)
       {
-        return nullptr;
+        hip_check(hipEventCreateWithFlags(&done_, hipEventDisableTiming | hipEventDisableSystemFence),
+                  "hipEventCreate chunk scratch");
       }
-      held_.emplace_back(stream, nullptr);
-      at = held_.end() - 1;
-    }
-    std::unique_ptr<DeviceBuffer> &buffer = at->second;
-    if (buffer == nullptr || buffer->bytes() < bytes)
-    {
-      buffer.reset(); // waits for launches that use it
-      try
+      drop();
+      const std::size_t roomy = std::max(bytes, std::min(growing_to, 2 * bytes));
+      for (const std::size_t size : {roomy, bytes})
       {
-        buffer = std::make_unique<DeviceBuffer>(std::max(bytes, growing_to));
-      }
-      catch (const OutOfMemory &)
-      {
+        if (hipMalloc(&buffer_, size) == hipSuccess)
+        {
+          size_ = size;
+          break;
+        }
         (void)hipGetLastError();
-        return nullptr;
+        buffer_ = nullptr;
+      }
+      if (buffer_ == nullptr)
+      {
+        return {nullptr, nullptr};
       }
     }
-    return buffer->raw();
+    hip_check(hipStreamWaitEvent(stream, done_, 0), "hipStreamWaitEvent chunk scratch");
+    ++taken_;
+    return {buffer_, done_};
+  }
+
+  std::size_t release_chunk_scratch()
+  {
+    ScratchList &list = scratch_list();
+    std::lock_guard<std::mutex> hold(list.lock);
+    std::size_t bytes = 0;
+    for (OwnedChunkScratch *scratch : list.all)
+    {
+      bytes += scratch->release();
+    }
+    return bytes;
   }
 
   const void *UploadBuffer::send_bytes(const void *host, std::size_t bytes, hipStream_t stream)
@@ -731,6 +834,12 @@ namespace mi
       // Memory the releaser has yet to give back may be what is short.
       (void)hipGetLastError();
       releaser_->wait_for(nullptr);
+      created = hipMemCreate(&handle, granules * granule_, &prop_, 0);
+    }
+    if ((created == hipErrorOutOfMemory || created == hipErrorMemoryAllocation) &&
+        release_chunk_scratch() > 0)
+    {
+      (void)hipGetLastError();
       created = hipMemCreate(&handle, granules * granule_, &prop_, 0);
     }
     hip_check(created, "hipMemCreate");

@@ -16,6 +16,7 @@
 #include "kernels.hpp"
 
 #include <array>
+#include <atomic>
 #include <condition_variable>
 #include <deque>
 #include <memory>
@@ -54,7 +55,11 @@ namespace mi
 
   std::string describe(PageKey key);
 
-  // Device memory owned by the library: RAII over hipMalloc.
+  // hipMalloc; where the device is out of memory, once more after the chunks'
+  // scratch is given back.
+  void *device_alloc(std::size_t bytes);
+
+  // Device memory owned by the library: RAII over device_alloc.
   class DeviceBuffer
   {
   public:
@@ -134,28 +139,46 @@ namespace mi
     std::vector<std::unique_ptr<DeviceBuffer>> outgrown_;
   };
 
-  // A buffer a stream, of one owner's, for launches that hand data to each
-  // other on that stream alone. Bounded: kMost streams (a buffer each, as
-  // large as its largest request); a further stream gets none, nor do the
-  // per-thread default streams, one handle for many streams, nor does a
-  // stream that is being captured, whose graph could be replayed beside
-  // other work of the owner's, nor a request the device has no memory for.
-  // Grown buffers and the owner's end give the old ones back, once the
-  // device is idle. take() is called with order() held.
-  class StreamBuffers final : public StreamScratch
+  // An owner's scratch for its chunks' attention: one buffer, as large as the
+  // largest request or, while the owner grows, up to twice that. A chunk on
+  // one stream waits for the chunk before it on another, whose work fills the
+  // device as well; the wait and the signal (an event that the last kernel
+  // completes) are free on a chunk's own stream. None for a stream that is
+  // being captured, whose graph could be replayed beside other chunks, nor
+  // where the device has no memory. A thread that captures another stream may
+  // ask: what it allocates and frees is in relaxed capture mode. Given back
+  // by the owner's end, by release_chunk_scratch, and when an allocation of
+  // this library's finds the device out of memory.
+  class OwnedChunkScratch final : public ChunkScratch
   {
   public:
+    OwnedChunkScratch();
+    ~OwnedChunkScratch();
+    OwnedChunkScratch(const OwnedChunkScratch &) = delete;
+    OwnedChunkScratch &operator=(const OwnedChunkScratch &) = delete;
     std::unique_lock<std::mutex> order() override
     {
       return std::unique_lock<std::mutex>(order_);
     }
-    void *take(hipStream_t stream, std::size_t bytes, std::size_t growing_to) override;
+    Taken take(hipStream_t stream, std::size_t bytes, std::size_t growing_to) override;
+    // The buffer given back once its last chunk is done; its bytes. 0 while
+    // a chunk is being launched.
+    std::size_t release();
+    std::size_t bytes() const { return size_; }
+    std::size_t taken() const { return taken_; } // chunks that were given it
 
   private:
-    static constexpr std::size_t kMost = 4;
+    void drop(); // with order() held
+
     std::mutex order_;
-    std::vector<std::pair<hipStream_t, std::unique_ptr<DeviceBuffer>>> held_;
+    void *buffer_ = nullptr;
+    hipEvent_t done_ = nullptr;
+    std::atomic<std::size_t> size_{0};
+    std::atomic<std::size_t> taken_{0};
   };
+
+  // Every owner's chunk scratch given back; the bytes.
+  std::size_t release_chunk_scratch();
 
   // Test hook: the next `n` granule maps fail as if the device were out of
   // memory, so rollback paths are exercised without exhausting real VRAM.
@@ -628,6 +651,7 @@ namespace mi
     bool masked(PageKey key) const { return flag(key, kMasked); }
     int page_tier(PageKey key) const { return allocator_.locate(key).tier; }
     const ShadowStore &shadows() const { return shadows_; }
+    const OwnedChunkScratch &chunk_scratch() const { return chunk_scratch_; }
     const std::optional<MoveRecord> &last_move() const { return last_move_; }
     const std::optional<BatchRecord> &last_batch() const { return last_batch_; }
     int page_tokens() const { return page_tokens_; }
@@ -726,8 +750,8 @@ namespace mi
     std::unique_ptr<DeviceBuffer> staging_;
     // The decode path's split partials and page statistics: this cache's own.
     OwnedWorkspace workspace_;
-    // A chunk's laid-out pages, a stream.
-    StreamBuffers chunk_scratch_;
+    // A chunk's laid-out pages.
+    OwnedChunkScratch chunk_scratch_;
     // Page statistics kept for fold_kept, every layer's (decode_kept_floats
     // a layer), and the step they belong to.
     OwnedWorkspace kept_;

@@ -200,6 +200,8 @@ SIGNATURES = {
     "mi_kv_page_tiers": ((_vp, _vp, _sz), C.c_int),
     "mi_kv_flags": ((_vp, _i, _vp, _sz), C.c_int),
     "mi_kv_info_get": ((_vp, C.POINTER(_KVInfo)), C.c_int),
+    "mi_kv_chunk_scratch": ((_vp, _szp, _szp), C.c_int),
+    "mi_release_chunk_scratch": ((_szp,), C.c_int),
     "mi_kv_birth_tier": ((_vp, _i, _i, _ip), C.c_int),
     "mi_kv_last_move": ((_vp, _ip, _ip, _szp, C.POINTER(C.c_double)), C.c_int),
     "mi_kv_last_batch": ((_vp, _ip, _szp, _szp, C.POINTER(C.c_double)), C.c_int),
@@ -967,6 +969,14 @@ def fail_next_granules(n: int) -> None:
     _check(lib.mi_debug_fail_next_granules(n))
 
 
+def release_chunk_scratch() -> int:
+    """Gives back the memory that caches keep for their next long chunk's
+    attention, once the chunks that use it are done; the bytes."""
+    out = C.c_size_t()
+    _check(lib.mi_release_chunk_scratch(C.byref(out)))
+    return out.value
+
+
 class KVPages:
     """The engine's KV cache on pages (kv_pages.h:105-412). Keeps its
     allocator alive."""
@@ -1013,6 +1023,14 @@ class KVPages:
     born_at_one_tier = property(lambda self: bool(self._info().born_at_one_tier))
     shadow_count = property(lambda self: self._info().shadow_count)
     shadow_bytes = property(lambda self: self._info().shadow_bytes)
+
+    @property
+    def chunk_scratch(self) -> tuple:
+        """How many chunks' attention laid the cache's pages out first, and
+        the bytes it keeps for the next one."""
+        chunks, held = C.c_size_t(), C.c_size_t()
+        _check(lib.mi_kv_chunk_scratch(self._h, C.byref(chunks), C.byref(held)))
+        return chunks.value, held.value
 
     def reserve(self, tokens: int) -> None:
         _check(lib.mi_kv_reserve(self._h, tokens))

@@ -92,51 +92,128 @@ def test_small_probabilities_keep_their_bits(heads, kv, hd, seq_q, high):
     assert error < 2.0**-11 + 2.0**-14 + 2.0**-16, error
 
 
-def test_captures_and_further_streams_take_the_staging_path():
-    """A captured launch and a fifth stream get no scratch and take the path
-    that needs none: the same attention, the graph replayed between the
-    program's own calls."""
+def chunk_call(layers=1, seq=P * 9 + 4, seq_q=144):
+    """A cache of `seq` positions and call(layer, out): its last seq_q
+    queries' attention; and each layer's attention and error bound."""
     m = mi()
     d = m.device
-    heads, kv, hd, seq, seq_q = 32, 8, 64, P * 9 + 4, 144
+    heads, kv, hd = 32, 8, 64
     rng = np.random.default_rng(9)
-    k, v, q = (normal(rng, seq, kv, hd), normal(rng, seq, kv, hd), normal(rng, seq_q, heads, hd))
+    q = normal(rng, seq_q, heads, hd)
     alloc, cache = pages_for(P, kv, hd, 0)
-    store_in_runs(cache, 0, k, v, [seq])
+    exact = []
+    for layer in range(layers):
+        k, v = normal(rng, seq, kv, hd), normal(rng, seq, kv, hd)
+        store_in_runs(cache, layer, k, v, [seq])
+        want, w = att.attention64(q, k, v)
+        exact.append((want, att.attention_bound(q, k, v, w)))
+    dq = put(q)
+
+    def call(layer, out, queries=seq_q):
+        cache.attention(layer, dq, None, None, out, queries, seq, heads, kv, hd, None, None, None,
+                        None)
+
+    def check(out, layer, what):
+        want, bound = exact[layer]
+        assert_attention_close(out.to_numpy().reshape(q.shape), want, what, bound)
+
+    for layer in range(layers):
+        call(layer, d.empty(q.size), 2)  # the page table is sent
     m.synchronize()
-    want, w = att.attention64(q, k, v)
-    bound = att.attention_bound(q, k, v, w)
-    dq, out = put(q), d.empty(q.size)
+    assert cache.chunk_scratch == (0, 0)
+    return (alloc, cache), call, lambda: d.empty(q.size), check
+
+
+def test_a_captured_chunk_takes_the_staging_path():
+    """A captured launch gets no scratch: the graph replayed between the
+    program's own calls, which do."""
+    m = mi()
+    d = m.device
+    (_, cache), call, empty, check = chunk_call()
+    out = empty()
     stream = m.Stream()
-
-    def call():
-        cache.attention(0, dq, None, None, out, seq_q, seq, heads, kv, hd, None, None, None, None)
-
     graph = m.Graph(stream)
     with graph.capture():
-        call()
+        call(0, out)
+    assert cache.chunk_scratch == (0, 0)
     for i in range(3):
         announce("chunk graph replay", i)
         d.random_half(out, 70 + i, 1.0)
         m.synchronize()
         graph.launch()
         stream.synchronize()
-        assert_attention_close(out.to_numpy().reshape(q.shape), want, f"replay {i}", bound)
+        check(out, 0, f"replay {i}")
         d.random_half(out, 90 + i, 1.0)
-        call()
-        assert_attention_close(out.to_numpy().reshape(q.shape), want, f"eager {i}", bound)
-    streams = [m.Stream() for _ in range(6)]
-    for i, s in enumerate(streams):
+        call(0, out)
+        check(out, 0, f"eager {i}")
+        assert cache.chunk_scratch[0] == i + 1
+
+
+def test_a_chunk_while_its_thread_captures_another_stream():
+    """The scratch's allocation and its return neither fail for a capture on
+    another stream nor spoil it."""
+    m = mi()
+    d = m.device
+    (_, cache), call, empty, check = chunk_call()
+    outs = [empty(), empty()]
+    side, stream = m.Stream(), m.Stream()
+    x, y = put(np.ones(64, np.float32)), put(np.ones(64, np.float32))
+    graph = m.Graph(stream)
+    with graph.capture():
+        d.add(x, y, x, 64)
+        m.set_stream(side)
+        for out in outs:
+            announce("chunk beside a capture")
+            call(0, out)
+            assert m.release_chunk_scratch() > 0
+        m.set_stream(stream)
+        d.add(x, y, x, 64)
+    side.synchronize()
+    for out in outs:
+        check(out, 0, "beside a capture")
+    assert cache.chunk_scratch == (2, 0)
+    for i in range(3):
+        graph.launch()
+        stream.synchronize()
+        np.testing.assert_array_equal(x.to_numpy(), np.full(64, 3.0 + 2 * i))
+
+
+def test_every_stream_lays_its_pages_out_in_the_one_scratch():
+    """Chunks of two layers on streams that come and go, more than any fixed
+    number, none waited for in between: each waits for the chunk before it."""
+    m = mi()
+    d = m.device
+    (_, cache), call, empty, check = chunk_call(layers=2, seq=P * 40 + 4)
+    outs = [empty() for _ in range(12)]
+    keep = [m.Stream() for _ in range(3)]
+    for i, out in enumerate(outs):
         announce("chunk stream", i)
-        d.random_half(out, i + 1, 1.0)
-        m.synchronize()
-        m.set_stream(s)
+        stream = keep[i % 3] if i % 2 else m.Stream()
+        m.set_stream(stream)
         try:
-            call()
+            call(i % 2, out)
         finally:
             m.set_stream(None)
-        s.synchronize()
-        assert_attention_close(out.to_numpy().reshape(q.shape), want, f"stream {i}", bound)
+    m.synchronize()
+    for i, out in enumerate(outs):
+        check(out, i % 2, f"call {i}")
+    assert cache.chunk_scratch[0] == len(outs)
+
+
+def test_the_scratch_is_given_back():
+    m = mi()
+    (_, cache), call, empty, check = chunk_call()
+    m.release_chunk_scratch()
+    out = empty()
+    call(0, out)
+    held = cache.chunk_scratch[1]
+    assert held > 0
+    assert m.release_chunk_scratch() == held
+    assert cache.chunk_scratch == (1, 0)
+    check(out, 0, "before")
+    call(0, out)
+    check(out, 0, "after")
+    assert cache.chunk_scratch == (2, held)
 
 
 def test_two_threads_chunks_on_one_stream_keep_their_own_layout():
