@@ -181,9 +181,9 @@ namespace mi
       int seal_block;
       // The workgroups a KV head's split launch holds at once (0: no bound).
       // When the live splits exceed it, busy_splits workgroups take the
-      // pages: each its own kWaves, and the pages past busy_splits * kWaves
-      // a wave each as a second page (kWaves * busy_splits on from its
-      // first); the splits past them are written as empty partials, so that
+      // pages: each its own split_waves, and the pages past busy_splits *
+      // split_waves a wave each as a second page (split_waves * busy_splits
+      // on from its first); the splits past them are written as empty partials, so that
       // readers of live_splits partials see the same layout.
       int busy_splits;
       // The row launch's work in the pages launch (decode_pages_kernel with
@@ -214,7 +214,10 @@ namespace mi
     __device__ inline u32x4 as_u32x4(half8 v) { return __builtin_bit_cast(u32x4, v); }
 
     // The launch's position, when it lives on the device: seq_k, the first
-    // chunk row (a decode step brings one) and the live bounds.
+    // chunk row (a decode step brings one) and the live bounds. kFew: the
+    // rule chooses the waves of a split by that position; otherwise a split
+    // takes all of a workgroup's.
+    template <bool kFew>
     __device__ inline void go_live(DecodeArgs &a)
     {
       if (a.live_seq_k != nullptr)
@@ -223,8 +226,16 @@ namespace mi
         a.seq_k = seq_k;
         a.start = seq_k - 1;
         a.live_pages = (seq_k + kPageTokens - 1) / kPageTokens;
-        a.split_waves = split_waves_of(a.split_rule, a.live_pages);
-        a.live_splits = (a.live_pages + a.split_waves - 1) / a.split_waves;
+        if constexpr (kFew)
+        {
+          a.split_waves = split_waves_of(a.split_rule, a.live_pages);
+          a.live_splits = (a.live_pages + a.split_waves - 1) / a.split_waves;
+        }
+        else
+        {
+          const int per_split = kWaves * a.pages_per_wave;
+          a.live_splits = (a.live_pages + per_split - 1) / per_split;
+        }
       }
     }
 
@@ -864,8 +875,11 @@ namespace mi
 
     // kCurrent: the row launch's work done here too (the DecodeArgs row_*
     // fields; one split layer, FP16 pages of a cache that does not seal, no
-    // key bias, no pack).
-    template <int HD, bool kBias, bool kCurrent = false>
+    // key bias, no pack). kFew: fewer than all of a workgroup's waves take a
+    // split's pages (split_waves); the others' code stays as it is without
+    // (a 1.5B step at 32K through the one kernel of both: 11.87 ms a run of
+    // eight against 11.72).
+    template <int HD, bool kBias, bool kFew, bool kCurrent = false>
     __global__ void __launch_bounds__(kThreads) decode_pages_kernel(DecodeArgs a)
     {
       constexpr int S = HD / 32;  // K steps of q.K^T
@@ -897,7 +911,7 @@ namespace mi
           return;
         }
       }
-      go_live(a);
+      go_live<kFew>(a);
       // (The key-bias kernel keeps one split a workgroup: its launches are
       // never bounded.)
       const int busy = !kBias && a.busy_splits > 0 && a.busy_splits < a.live_splits
@@ -921,9 +935,10 @@ namespace mi
       const unsigned long long *table = a.table + layer * a.table_stride;
       const std::uint8_t *tiers = a.tiers != nullptr ? a.tiers + layer * a.table_stride : nullptr;
       const int own = a.causal ? (a.seq_k - 1) / kPageTokens : -1;
+      const int split_waves = kFew ? a.split_waves : kWaves;
       // (An idle wave starts past the last page.)
-      const int p0 = (split * a.split_waves + wave) * a.pages_per_wave +
-                     (wave < a.split_waves ? 0 : a.live_pages);
+      const int p0 = (split * split_waves + wave) * a.pages_per_wave +
+                     (!kFew || wave < split_waves ? 0 : a.live_pages);
       // The wave's pages: p0 and the next pages_per_wave - 1 (several a
       // wave), or p0 and every split_waves * busy pages on (the pages past the
       // busy splits).
@@ -932,7 +947,7 @@ namespace mi
       {
         if (a.pages_per_wave == 1)
         {
-          p_step = a.split_waves * busy;
+          p_step = split_waves * busy;
           p_count = INT_MAX;
         }
       }
@@ -2050,7 +2065,8 @@ namespace mi
       }
     }
 
-    template <int HD, bool Streamed>
+    // kFew: a live launch whose split the rule chooses (go_live).
+    template <int HD, bool Streamed, bool kFew = false>
     __global__ void __launch_bounds__(kCombineThreads) decode_combine_kernel(const DecodeArgs args)
     {
       if constexpr (!Streamed)
@@ -2067,7 +2083,7 @@ namespace mi
       DecodeArgs a = args;
       // Fixed splits unless the streaming kernel wrote the partials: the
       // per-layer form carries none of the streaming geometry's code.
-      go_live(a);
+      go_live<kFew>(a);
       const auto splits_of = [&](int li, int kvh) {
         return Streamed ? group_splits(a, li, kvh) : a.live_splits;
       };
@@ -2266,7 +2282,8 @@ namespace mi
               fold_partial(top, sum, ml[j][k].x, ml[j][k].y);
             }
           }
-          // More than 128 splits only when several layers share a launch.
+          // More than 128 splits: several layers in a launch, or few pages a
+          // split of one layer of few KV heads.
           const float2 *mls = head_ml(h);
           for (int sp = lane + 128; sp < splits[j]; sp += 64)
           {
@@ -2327,6 +2344,14 @@ namespace mi
       return {cus * 5 / 8 / kv_heads * 2, cus / kv_heads * 4};
     }
 
+    // Whether any position from `seq_k` to the last of `pages` pages makes
+    // more than one split of fewer than all of a workgroup's waves.
+    bool few_waves_from(const SplitRule &r, int seq_k, int pages)
+    {
+      const int least = (std::max(seq_k, 1) + kPageTokens - 1) / kPageTokens;
+      return split_waves_of(r, least) < kWaves && pages > split_waves_of(r, pages);
+    }
+
     bool aligned16(const void *p) { return (reinterpret_cast<std::uintptr_t>(p) & 15u) == 0; }
 
     // Waves of the head_dim-64 pages kernel (a wave a page of one KV head)
@@ -2347,7 +2372,7 @@ namespace mi
       }
       int blocks = 0;
       hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &blocks, reinterpret_cast<const void *>(decode_pages_kernel<64, false>),
+                    &blocks, reinterpret_cast<const void *>(decode_pages_kernel<64, false, false>),
                     kThreads, lds),
                 "hipOccupancyMaxActiveBlocksPerMultiprocessor decode");
       int cus = 0;
@@ -2602,6 +2627,20 @@ namespace mi
     }
     d.live_pages = pages;
     d.live_splits = ls.split && !streaming ? (pages + d.split_waves - 1) / d.split_waves : d.splits;
+    // The kernel of few waves a split: a live launch takes it where any of its
+    // positions may need it, the key bias at head_dim 128 and the row's work
+    // where their own pages do (one split holds them all either way where
+    // they are no more than its waves). Any other split launch takes it
+    // always: at eight waves a split it is the faster there (28 layers of the
+    // 1.5B shape at 32,768: 405 -> 403 us a token, 24 of the 0.5B with the key
+    // bias 308 -> 301; the 1.5B with it 493 -> 501, its row launch at 40
+    // positions 287 -> 294).
+    const bool few_live = ls.live_seq_k != nullptr && few_waves_from(d.split_rule, ls.least_seq_k, pages);
+    const bool few_pages = d.split_waves < kWaves && d.live_splits > 1;
+    const bool few = ls.live_seq_k != nullptr ? few_live
+                     : row != nullptr || (d.k_bias != nullptr && a.head_dim == 128)
+                         ? few_pages
+                         : ls.split && !streaming;
     // head_dim 64 with an even number of KV heads and no key bias (the
     // Llama shapes): two KV heads a wave, as one 128-channel unit, so that a
     // launch has half the waves, each with a unit of the size the kernel's
@@ -2696,53 +2735,39 @@ namespace mi
                          dim3(kCombineThreads), 0, stream, d);
       hip_check(hipGetLastError(), "decode combine kernel launch");
     };
-    if (row != nullptr)
+    // The kernels of a shape, by how its launches split.
+    const auto go = [&](auto hd_tag, auto pages_hd_tag, auto bias_tag, auto current_tag) {
+      constexpr int kHD = decltype(hd_tag)::value;
+      constexpr int kPagesHD = decltype(pages_hd_tag)::value;
+      constexpr bool kBias = decltype(bias_tag)::value;
+      constexpr bool kCurrent = decltype(current_tag)::value;
+      run(few ? decode_pages_kernel<kPagesHD, kBias, true, kCurrent>
+              : decode_pages_kernel<kPagesHD, kBias, false, kCurrent>,
+          decode_stream_kernel<kHD>,
+          few_live ? decode_combine_kernel<kHD, false, true> : decode_combine_kernel<kHD, false>,
+          decode_combine_kernel<kHD, true>, kHD, stream_kernel_lds<kHD>(), kPagesHD);
+    };
+    using Hd64 = std::integral_constant<int, 64>;
+    using Hd128 = std::integral_constant<int, 128>;
+    const std::true_type yes;
+    const std::false_type no;
+    const bool bias = d.k_bias != nullptr;
+    if (a.head_dim == 128)
     {
-      if (a.head_dim == 128)
-      {
-        run(decode_pages_kernel<128, false, true>, decode_stream_kernel<128>,
-            decode_combine_kernel<128, false>, decode_combine_kernel<128, true>, 128,
-            stream_kernel_lds<128>(), 128);
-      }
-      else
-      {
-        run(decode_pages_kernel<64, false, true>, decode_stream_kernel<64>,
-            decode_combine_kernel<64, false>, decode_combine_kernel<64, true>, 64,
-            stream_kernel_lds<64>(), 64);
-      }
-    }
-    else if (a.head_dim == 128)
-    {
-      if (d.k_bias != nullptr)
-      {
-        run(decode_pages_kernel<128, true>, decode_stream_kernel<128>,
-            decode_combine_kernel<128, false>, decode_combine_kernel<128, true>, 128,
-            stream_kernel_lds<128>(), 128);
-      }
-      else
-      {
-        run(decode_pages_kernel<128, false>, decode_stream_kernel<128>,
-            decode_combine_kernel<128, false>, decode_combine_kernel<128, true>, 128,
-            stream_kernel_lds<128>(), 128);
-      }
+      row != nullptr ? go(Hd128{}, Hd128{}, no, yes)
+      : bias         ? go(Hd128{}, Hd128{}, yes, no)
+                     : go(Hd128{}, Hd128{}, no, no);
     }
     else if (packed)
     {
       // The pack's unit is 128 channels; each head's output is its own 64.
-      run(decode_pages_kernel<128, false>, decode_stream_kernel<64>,
-          decode_combine_kernel<64, false>, decode_combine_kernel<64, true>, 64,
-          stream_kernel_lds<64>(), 128);
-    }
-    else if (d.k_bias != nullptr)
-    {
-      run(decode_pages_kernel<64, true>, decode_stream_kernel<64>, decode_combine_kernel<64, false>,
-          decode_combine_kernel<64, true>, 64, stream_kernel_lds<64>(), 64);
+      go(Hd64{}, Hd128{}, no, no);
     }
     else
     {
-      run(decode_pages_kernel<64, false>, decode_stream_kernel<64>,
-          decode_combine_kernel<64, false>, decode_combine_kernel<64, true>, 64,
-          stream_kernel_lds<64>(), 64);
+      row != nullptr ? go(Hd64{}, Hd64{}, no, yes)
+      : bias         ? go(Hd64{}, Hd64{}, yes, no)
+                     : go(Hd64{}, Hd64{}, no, no);
     }
   }
 
@@ -2793,8 +2818,12 @@ namespace mi
     d.mass_blocks = (pages + 63) / 64;
     const int blocks_a_head = f.head_dim / (4 * kQuads);
     d.block_base = f.heads * blocks_a_head;
-    const auto kernel = f.head_dim == 128 ? decode_combine_kernel<128, false>
-                                          : decode_combine_kernel<64, false>;
+    const bool few = f.live_seq_k != nullptr && few_waves_from(d.split_rule, f.least_seq_k, pages);
+    const auto kernel = f.head_dim == 128
+                            ? (few ? decode_combine_kernel<128, false, true>
+                                   : decode_combine_kernel<128, false>)
+                            : (few ? decode_combine_kernel<64, false, true>
+                                   : decode_combine_kernel<64, false>);
     hipLaunchKernelGGL(kernel, dim3(d.mass_blocks, f.layers), dim3(kCombineThreads), 0, stream, d);
     hip_check(hipGetLastError(), "decode fold kernel launch");
   }

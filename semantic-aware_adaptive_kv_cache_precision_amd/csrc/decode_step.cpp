@@ -122,7 +122,7 @@ namespace mi
     }
   }
 
-  void DecodeStep::enqueue_step(int max_seq_k, hipStream_t stream)
+  void DecodeStep::enqueue_step(int least_seq_k, int max_seq_k, hipStream_t stream)
   {
     const ModelShape &s = shape_;
     const int q_width = s.heads * s.head_dim;
@@ -185,7 +185,7 @@ namespace mi
       launch_qkv_step(qkv, stream);
       cache_.attention_step(l, qk, key_bias_ ? w.k_b : nullptr, &rope_, attended,
                             state + kStepSeqK, max_seq_k, s.heads, s.kv_heads, s.head_dim,
-                            qk + q_width, v, kept, &target);
+                            qk + q_width, v, kept, &target, least_seq_k);
       ProjectArgs o{};
       o.segments = 1;
       o.seg[0] = {w.o_w, nullptr, residual, s.hidden};
@@ -232,7 +232,7 @@ namespace mi
     {
       cache_.fold_step(kept, state + kStepSeqK, max_seq_k, s.heads, s.kv_heads, s.head_dim,
                        score_every_, scores_->layer_scores(0), scores_->max_pages(),
-                       scores_->alpha());
+                       scores_->alpha(), least_seq_k);
       ++launches;
     }
     launch_advance(best_value_->as<float>(), best_index_->as<int>(), head_blocks_, s.vocab, state,
@@ -265,7 +265,7 @@ namespace mi
     hip_check(hipDeviceSynchronize(), "hipDeviceSynchronize before capture");
   }
 
-  void DecodeStep::capture(int max_seq_k)
+  void DecodeStep::capture(int least_seq_k, int max_seq_k)
   {
     prepare_launches(max_seq_k);
     if (exec_ != nullptr)
@@ -280,7 +280,7 @@ namespace mi
               "hipStreamBeginCapture step");
     try
     {
-      enqueue_step(max_seq_k, stream_);
+      enqueue_step(least_seq_k, max_seq_k, stream_);
     }
     catch (...)
     {
@@ -305,13 +305,13 @@ namespace mi
     require(steps > 0 && position >= 0, "a run takes at least one step from a position >= 0");
     require(tokens != nullptr, "a run writes its tokens to host memory");
     const int end = position + steps;
-    // The run's pages, then a graph for the most positions it attends (or,
+    // The run's pages, then a graph for the positions it attends (or,
     // eager, the same launches made from the host a step at a time).
     cache_.reserve(end);
     size_buffers(steps);
     if (graphed)
     {
-      capture(end);
+      capture(position + 1, end);
     }
     else
     {
@@ -336,7 +336,7 @@ namespace mi
       {
         for (int i = 0; i < steps; ++i)
         {
-          enqueue_step(end, stream_);
+          enqueue_step(position + 1, end, stream_);
         }
       }
       catch (...)

@@ -114,8 +114,8 @@ namespace mi
   private:
     void size_buffers(int steps);
     void prepare_launches(int max_seq_k);
-    void capture(int max_seq_k);
-    void enqueue_step(int max_seq_k, hipStream_t stream);
+    void capture(int least_seq_k, int max_seq_k);
+    void enqueue_step(int least_seq_k, int max_seq_k, hipStream_t stream);
 
     KVPages &cache_;
     ModelShape shape_;

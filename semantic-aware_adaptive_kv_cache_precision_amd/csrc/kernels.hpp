@@ -431,8 +431,10 @@ namespace mi
     // A decode whose position lives on the device (one layer, split, not
     // several layers at once): seq_k is read from *live_seq_k when the
     // kernels run, and AttentionArgs::seq_k is the most it may be, which
-    // sizes the launch and the strides.
+    // sizes the launch and the strides; least_seq_k the least (0: unknown),
+    // which tells whether the launch may be split over few waves.
     const int *live_seq_k;
+    int least_seq_k;
     // With a live position: the step's page seal, done by one more
     // workgroup of the combine when *seal->position is its page's last row
     // (the page quantised, or copied at FP16, from the open page's rows and
@@ -480,8 +482,10 @@ namespace mi
     float alpha;
     // With the position on the device: seq_k read from *live_seq_k, `seq_k`
     // above the most it may be (the kept layout's size); the fold runs only
-    // where that seq_k is a multiple of score_every.
+    // where that seq_k is a multiple of score_every. least_seq_k as the
+    // decodes' that kept the statistics.
     const int *live_seq_k;
+    int least_seq_k;
     int score_every;
   };
   std::size_t decode_kept_floats(int heads, int kv_heads, int seq_k);

@@ -1544,7 +1544,7 @@ namespace mi
   void KVPages::attention_step(int layer, const void *q, const void *k_bias, const RopeTable *rope,
                                void *out, const int *live_seq_k, int max_seq_k, int heads,
                                int kv_heads, int head_dim, const void *keys, const void *values,
-                               float *keep, const StepStore *seal)
+                               float *keep, const StepStore *seal, int least_seq_k)
   {
     require_layer(layer);
     if (static_cast<std::size_t>(kv_heads) * head_dim != kv_width_)
@@ -1600,6 +1600,7 @@ namespace mi
     ls.split = true;
     ls.layers = 1;
     ls.live_seq_k = live_seq_k;
+    ls.least_seq_k = least_seq_k;
     ls.seal = seal;
     if (keep != nullptr)
     {
@@ -1615,7 +1616,7 @@ namespace mi
 
   void KVPages::fold_step(float *keep, const int *live_seq_k, int max_seq_k, int heads,
                           int kv_heads, int head_dim, int score_every, float *scores,
-                          long long scores_stride, float alpha)
+                          long long scores_stride, float alpha, int least_seq_k)
   {
     if (keep == nullptr || live_seq_k == nullptr || score_every < 1)
     {
@@ -1633,6 +1634,7 @@ namespace mi
     f.scores_stride = scores_stride;
     f.alpha = alpha;
     f.live_seq_k = live_seq_k;
+    f.least_seq_k = least_seq_k;
     f.score_every = score_every;
     launch_decode_fold(f, runtime_stream());
   }

@@ -594,7 +594,8 @@ namespace mi
     // completes); attention_step decodes one layer at seq_k = *live_seq_k,
     // its launch sized for max_seq_k, keeping its statistics in `keep` (a
     // DecodeFold's layout for every layer at max_seq_k) when keep is not
-    // null; fold_step folds the kept statistics into the scores where seq_k
+    // null, and least_seq_k the least position it may run at (0: unknown);
+    // fold_step folds the kept statistics into the scores where seq_k
     // is a multiple of score_every. prepare_step readies the tables and
     // scratch for max_seq_k beforehand, so that the launches allocate and
     // upload nothing; the pages up to max_seq_k must be reserved, and no
@@ -632,10 +633,10 @@ namespace mi
     void attention_step(int layer, const void *q, const void *k_bias, const RopeTable *rope,
                         void *out, const int *live_seq_k, int max_seq_k, int heads,
                         int kv_heads, int head_dim, const void *keys, const void *values,
-                        float *keep, const StepStore *seal = nullptr);
+                        float *keep, const StepStore *seal = nullptr, int least_seq_k = 0);
     void fold_step(float *keep, const int *live_seq_k, int max_seq_k, int heads, int kv_heads,
                    int head_dim, int score_every, float *scores, long long scores_stride,
-                   float alpha);
+                   float alpha, int least_seq_k = 0);
     void stored_on_device(int end);
     void downgrade(int layer, int page, int target);
     void upgrade(int layer, int page, int target);

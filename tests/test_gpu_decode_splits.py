@@ -1,8 +1,10 @@
 """One layer's decode where its split changes: a quarter of a workgroup's
-waves a split, half of them up to a workgroup a CU, all of them past it. Outputs and masses against
-the float64 oracle on both sides; a launch sized for a long context with its
-seq_k on the device, and the statistics kept for a later fold, to the bits of
-the plain launch at every seq_k."""
+waves a split, half of them up to a workgroup a CU, all of them past it. Outputs
+and masses against the float64 oracle on both sides; a launch sized for a long
+context with its seq_k on the device, and the statistics kept for a later fold,
+to the bits of the plain launch at every seq_k; a run of steps across a change
+to the bits of the steps one by one, whose kernels are chosen by their own
+positions."""
 
 import numpy as np
 import pytest
@@ -10,6 +12,8 @@ import pytest
 from conftest import announce, assert_attention_close, fp16_exact
 from oracle import attention as att
 from oracle import ewma
+from test_gpu_decode_step import (context_rows, make_cache, make_weights, prefill, small_shape,
+                                  tier_map_for, upload_weights)
 from test_gpu_kv_pages import LAYERS, mi, normal, page_sizes, put, sealed_pages
 
 pytestmark = pytest.mark.gpu
@@ -86,3 +90,36 @@ def test_decode_on_both_sides_of_the_split(heads, kv, hd, bias):
         assert_attention_close(outs[0].astype(np.float64).reshape(1, heads, hd), want,
                                f"seq {seq}", bound)
         np.testing.assert_allclose(got[0].sum(1), 1.0, rtol=1e-3)
+
+
+@pytest.mark.parametrize("start", [
+    60,    # from two pages, one split either way, to three
+    1020,  # from 32 pages, splits of four, to 33, splits of eight
+])
+@pytest.mark.parametrize("bias", [False, True])
+def test_a_run_across_a_change_of_split_is_its_steps(start, bias):
+    """32 KV heads: splits of two up to 10 pages, of four up to 32 (256 CUs).
+    (Steps launched from the host: the launches a graph would hold.)"""
+    m = mi()
+    d = m.device
+    s = small_shape(heads=32, kv_heads=32, head_dim=64)
+    rng = np.random.default_rng(start)
+    dev = upload_weights(make_weights(rng, s, bias))
+    rows = context_rows(rng, s, start)
+    n, made = 9, []
+    for runs in ([n], [1] * n):
+        alloc, cache = make_cache(s, tier_map_for(s, 64))
+        prefill(cache, s, rows)
+        scores = d.ImportanceScores(s["layers"], 40)
+        step = d.DecodeStep(cache, s, dev["embed"], dev["final_norm"], dev["head"], dev["layers"],
+                            scores, 1)
+        token, at, tokens = 3, start, []
+        for k in runs:
+            announce("steps across a split", start, bias, at, k)
+            out, _ = step.run(token, at, k, graphed=False)
+            tokens += [int(t) for t in out]
+            token, at = tokens[-1], at + k
+        made.append((tokens, step.logits(), scores.download(), alloc, cache, step))
+    assert made[0][0] == made[1][0]
+    np.testing.assert_array_equal(made[0][1], made[1][1])
+    np.testing.assert_array_equal(made[0][2], made[1][2])
