@@ -499,9 +499,8 @@ namespace mi
   {
     kHalf,       // out fp16 = acc + bias (fp32, one rounding)
     kAccumulate, // out fp32 += acc
-    kFloat,      // out fp32 = acc
     kSwiglu,     // seg[0] gate, seg[1] up: seg[0].out fp16 = silu(g) u
-    kLogits,     // out fp32 = acc, and each block's best (value, index)
+    kLogits,     // out fp32 = acc, and with best_value each block's best (value, index)
   };
   constexpr int kProjectSegments = 3;
   struct ProjectSegment

@@ -245,7 +245,7 @@ namespace mi
       }
       return;
     }
-    if (project_row(accumulate ? ProjectMode::kAccumulate : ProjectMode::kFloat, x, weight,
+    if (project_row(accumulate ? ProjectMode::kAccumulate : ProjectMode::kLogits, x, weight,
                     nullptr, out, rows, in_features, out_features, stream))
     {
       return;

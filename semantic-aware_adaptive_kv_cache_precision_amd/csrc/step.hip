@@ -410,9 +410,6 @@ namespace mi
           *out = *out + dot;
           break;
         }
-        case ProjectMode::kFloat:
-          static_cast<float *>(sg.out)[row] = dot;
-          break;
         case ProjectMode::kSwiglu:
         {
           const float gv = h2f(to_half(dot));
@@ -449,7 +446,7 @@ namespace mi
           turn(a, b, 1);
         }
       }
-      if (p.mode == ProjectMode::kLogits)
+      if (p.best_value != nullptr)
       {
         // The workgroup's best logit, for the advance to choose from (parts
         // other than the first hold no candidate).
@@ -848,9 +845,11 @@ namespace mi
                               " needs 16-byte aligned weights, rows and an output");
       }
     }
-    if (p.mode == ProjectMode::kLogits && (p.best_value == nullptr || p.best_index == nullptr))
+    if ((p.best_value == nullptr) != (p.best_index == nullptr) ||
+        (p.best_value != nullptr && p.mode != ProjectMode::kLogits))
     {
-      throw InvalidArgument("the head's projection keeps each block's best logit");
+      throw InvalidArgument("each block's best logit, its value and its index, is the head's "
+                            "projection's to keep");
     }
     // The input in LDS: in fp16 values.
     if (static_cast<std::size_t>(p.in) * 2 > 64 * 1024)
@@ -861,7 +860,7 @@ namespace mi
     const ProjectPlan plan = plan_projection(p);
     // Each workgroup of the head writes its best logit: the arrays must hold
     // one an entry a workgroup.
-    if (p.mode == ProjectMode::kLogits && plan.blocks > p.best_count)
+    if (p.best_value != nullptr && plan.blocks > p.best_count)
     {
       throw InvalidArgument("the head's projection runs " + std::to_string(plan.blocks) +
                             " workgroups; its best arrays hold " + std::to_string(p.best_count));
