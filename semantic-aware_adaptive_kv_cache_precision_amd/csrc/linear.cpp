@@ -20,7 +20,9 @@
 // hipBLASLt's tiles of 16 rows took 7.4 us for a 1.5B layer's q, k, v and
 // output projections, 8.5 for gate and up and 15.2 for down, where it takes
 // 3.5 to 4.5, 8.0 and 7.8 (a layer's row through the operator calls: 132 ->
-// 85 us). More rows share a tile's weights and stay with hipBLASLt.
+// 85 us). Many short weight rows leave its waves little to ask for each and
+// stay with hipBLASLt (row_pays), as do more rows, which share a tile's
+// weights.
 // Each shape's descriptors and algorithm are looked up once and kept. The
 // workspace is fixed and generous, so an algorithm that splits the reduction
 // reduces its partials in fp32 in the workspace rather than in the output
@@ -175,11 +177,25 @@ namespace mi
                  "hipblasLtMatmul");
     }
 
+    // Whether one row's projection is faster by the matrix-vector kernel (GPU
+    // times in a graph over weights not in the caches, hipBLASLt's first): a
+    // wave takes a weight row, so rows of at least 1,536 values keep it busy
+    // at any number of them (1,536 x 256 6.8 us against 3.5, x 8,960 10.7 / 8.0,
+    // x 151,936 166 / 88; 4,096 x 14,336 26.2 / 24.5); shorter ones while they
+    // are few: 896 x 4,096 7.1 / 5.0 and x 14,336 9.1 / 8.9, but x 151,936
+    // 54 / 61; 512 x 4,096 5.5 / 4.4, x 65,536 17.0 / 21.8; 256 x 1,024 3.9 / 3.3,
+    // x 32,768 8.2 / 10.7; 64 x 128 4.3 / 2.7, x 151,936 12.2 / 36.2.
+    bool row_pays(int in_features, int out_features)
+    {
+      return in_features >= 1536 || out_features / (in_features >= 512 ? 8 : 4) <= in_features;
+    }
+
     // y = x W^T of one row through the matrix-vector kernel, when it takes it.
     bool project_row(ProjectMode mode, const void *x, const void *weight, const void *bias,
                      void *out, int rows, int in_features, int out_features, hipStream_t stream)
     {
-      if (rows != 1 || !project_applies(x, weight, in_features))
+      if (rows != 1 || !project_applies(x, weight, in_features) ||
+          !row_pays(in_features, out_features))
       {
         return false;
       }

@@ -25,6 +25,8 @@ def check(got, x, w, add, half):
 
 @pytest.mark.parametrize("n_in,n_out", [
     (8, 1), (8, 5), (504, 7), (512, 4), (520, 1000), (1536, 256), (1536, 8960), (4096, 33),
+    (64, 259), (64, 260), (504, 2020), (512, 4103), (512, 4104),  # many short rows: hipBLASLt's
+    (1528, 12240), (1536, 12300),
     (4104, 9),       # the first length split over four waves
     (8960, 130), (16384, 6), (16392, 3), (32768, 5),
     (32776, 3), (12, 6), (1000, 3),   # hipBLASLt's: too long, not a multiple of 8 (1000 is)
@@ -70,14 +72,15 @@ def test_rows_off_their_alignment_and_several_rows_agree_with_one():
         check(got[1 if rows == 3 else 0], x[1], w, np.zeros(n_out), True)
 
 
-def test_logits_of_one_row():
+@pytest.mark.parametrize("hidden", [64, 1536])  # hipBLASLt's, and the matrix-vector kernel's
+def test_logits_of_one_row(hidden):
     """The head's fp32 logits of one row among several, and its argmax."""
     m = mi()
     d = m.device
-    hidden, vocab = 64, 5003
+    vocab = 5003
     rng = np.random.default_rng(6)
     x = fp16_exact(rng.standard_normal((4, hidden)))
-    w = fp16_exact(rng.standard_normal((vocab, hidden)) / 8)
+    w = fp16_exact(rng.standard_normal((vocab, hidden)) / np.sqrt(hidden))
     scratch = d.empty(d.scratch_elements(1, vocab))
     announce("logits of one row")
     got = d.logits(put(x), put(w), scratch, 2, 1, hidden, vocab)
