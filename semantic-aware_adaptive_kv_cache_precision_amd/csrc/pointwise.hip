@@ -47,8 +47,10 @@ namespace mi
     }
 
     // RoPE with the angle formed per pair in fp64: a thread a rotation pair
-    // of every (token, head) row, the grid striding over them. For a few
-    // tokens: one row of 12 heads takes 2.7 us, 3.1 through rope_tokens_kernel.
+    // of every (token, head) row, the grid striding over them. For few pairs
+    // (one row of 12 heads takes 2.7 us, 3.1 through rope_tokens_kernel) and
+    // for few heads, which have few angles to share (8,192 tokens of one head
+    // of 64: 5.1 us against 13.2; of four 14.2 and 14.4, of six 20.4 and 15.4).
     __global__ void rope_kernel(const std::uint16_t *__restrict__ x,
                                 const std::int32_t *__restrict__ positions,
                                 std::uint16_t *__restrict__ out, int heads, int head_dim,
@@ -333,7 +335,9 @@ namespace mi
       return;
     }
     const std::size_t pairs = static_cast<std::size_t>(seq) * heads * (head_dim / 2);
-    if (pairs <= 32768)
+    // A workgroup a token pays where a token's rows have pairs to fill it:
+    // five heads of 64 channels' (rope_kernel's comment).
+    if (pairs <= 32768 || heads * (head_dim / 2) < 160)
     {
       hipLaunchKernelGGL(rope_kernel, dim3(grid_for(pairs, 256)), dim3(256), 0, stream,
                          static_cast<const std::uint16_t *>(x), positions,

@@ -47,6 +47,7 @@ def test_a_long_store_is_its_pages_stored_one_at_a_time(kv, hd, runs):
 @pytest.mark.parametrize("seq,heads,hd", [
     (32, 32, 64), (33, 32, 64),    # the last token by token a pair, the first by workgroups
     (5, 3, 6), (700, 3, 34), (70, 2, 514), (40, 5, 1030),
+    (600, 4, 64), (600, 5, 64), (600, 2, 128), (600, 3, 128),  # few heads: a thread a pair
 ])
 def test_rope_of_many_tokens_is_each_tokens(seq, heads, hd):
     m = mi()
