@@ -16,30 +16,35 @@ P = 32
 
 
 @pytest.mark.parametrize("kv,hd,runs", [
-    (8, 64, [64]),                 # two pages: job by job
-    (8, 64, [65]),                 # the shortest run, and a row over
-    (2, 128, [7, 120, 33]),        # a first page begun by an earlier store
-    (2, 64, [31, 1, 96, 130]),
+    (8, 64, [65]),                 # few pages: job by job
+    (8, 64, [P * 24]),             # the most pages as jobs
+    (8, 64, [P * 24 + 1]),         # the shortest run, and a row over
+    (2, 128, [7, P * 24 - 6, 33]), # a first page begun by an earlier store
+    (2, 64, [31, 1, 96, P * 25]),
     (2, 64, [P * 256 + 5]),        # a full launch of pages
     (2, 64, [3, P * 257 + 40]),    # one page into a second launch
     (1, 64, [200]),                # not a register-quantiser shape
 ])
 def test_a_long_store_is_its_pages_stored_one_at_a_time(kv, hd, runs):
+    """Every page, the last of which a further store completes: its first
+    rows have waited in an open page."""
     seq = sum(runs)
+    pages = -(-seq // P)
     rng = np.random.default_rng(seq)
-    k, v = normal(rng, seq, kv, hd), normal(rng, seq, kv, hd)
-    tmap = [[(1, 0, 3, 2)[(p + l) % 4] for p in range(seq // P + 1)] for l in range(LAYERS)]
+    k, v = normal(rng, pages * P, kv, hd), normal(rng, pages * P, kv, hd)
+    tmap = [[(1, 0, 3, 2)[(p + l) % 4] for p in range(pages)] for l in range(LAYERS)]
     made = []
-    for pieces in (runs, [min(P, seq - at) for at in range(0, seq, P)]):
+    for pieces in (list(runs), [min(P, seq - at) for at in range(0, seq, P)]):
         alloc, cache = pages_for(P, kv, hd, 0, tier_map=tmap, always_seal=True,
-                                 capacity=(seq // P + 1) * LAYERS + 8)
+                                 capacity=pages * LAYERS + 8)
         announce("store", kv, hd, pieces[:4])
-        cache.reserve(seq)
+        cache.reserve(pages * P)
         at = 0
-        for n in pieces:
-            cache.store(1, put(k[at:at + n]), put(v[at:at + n]), at, n)
+        for n in pieces + [pages * P - seq]:
+            if n > 0:
+                cache.store(1, put(k[at:at + n]), put(v[at:at + n]), at, n)
             at += n
-        made.append([alloc.read(1, p) for p in range(seq // P)])
+        made.append([alloc.read(1, p) for p in range(pages)])
     for p, (a, b) in enumerate(zip(*made)):
         np.testing.assert_array_equal(a, b, err_msg=f"page {p}")
 
