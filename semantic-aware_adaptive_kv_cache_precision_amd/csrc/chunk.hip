@@ -875,12 +875,43 @@ namespace mi
                                  : run<64, 2, 2, false, 2>(args, work, done, stream);
     }
 
+    // Whether the layout, a launch and the pages' bytes written and read as
+    // FP16, costs less than dequantising and staging each page once a query
+    // block. (Microseconds staged / laid out, mixed tiers, 8 to 64 heads in
+    // groups of 1 to 16, heads / KV heads x queries after positions before.)
+    bool laying_out_pays(const AttentionArgs &a)
+    {
+      // Fewer rows a KV head than a workgroup takes at head_dim 128: every
+      // page is staged once either way (32/32 x 64 after 8,000 at head_dim
+      // 128: 80 / 83).
+      if (static_cast<long long>(a.seq_q) * (a.heads / a.kv_heads) < block_rows(1))
+      {
+        return false;
+      }
+      const long long rows = static_cast<long long>(a.seq_q) * a.heads;
+      const bool wide = a.head_dim == 128;
+      // Over many keys, once the rows keep the device busy: at head_dim 64
+      // 8/8 x 128 after 8,000 33 / 38, x 256 60 / 43, 32/16 x 64 51 / 53, 14/2
+      // x 160 after 2,000 with the key bias 32 / 29. At 128 8/8 x 128 after
+      // 8,000 40 / 45, 8/1 x 192 after 3,000 35 / 31.
+      if (a.seq_k > 2048)
+      {
+        return wide ? rows >= 1536 : rows > 2048;
+      }
+      // Over few, where the layout's and the splits' launches weigh more: at
+      // head_dim 64 14/2 x 256 after 500 with the key bias 31 / 35, 8/8 x 513
+      // after 100 with it 42 / 45, 32/16 x 160 after 500 39 / 35; at 128 8/1 x
+      // 257 after 500 29 / 31, 14/2 x 160 28.2 / 28.6, 12/2 x 192 30.1 / 29.6.
+      // Over fewer than 128 32/8 x 96 alone 11.8 / 13.3.
+      return a.seq_k >= 128 && rows >= (wide ? 2304 : 4608);
+    }
+
   } // namespace
 
   bool chunk_applies(const KVSource &kv, const AttentionArgs &a)
   {
-    return a.seq_q >= kChunkQueries * (a.head_dim == 64 ? 2 : 1) && kv.layout != Layout::kContiguous &&
-           a.heads / a.kv_heads <= block_rows(1) && prefill_applies(kv, a);
+    return kv.layout != Layout::kContiguous && a.kv_heads > 0 && a.heads % a.kv_heads == 0 &&
+           a.heads / a.kv_heads <= block_rows(1) && laying_out_pays(a) && prefill_applies(kv, a);
   }
 
   std::size_t chunk_workspace_bytes(const KVSource &kv, const AttentionArgs &a)

@@ -388,15 +388,9 @@ namespace mi
   void launch_prefill(const KVSource &kv, const AttentionArgs &a, hipStream_t stream);
 
   // The chunk path over laid-out pages (chunk.hip): what prefill_applies
-  // takes, of a paged or sealing cache and at least kChunkQueries queries at
-  // head_dim 128, twice as many at 64, whose pages cost the staging kernel
-  // half as much. 64 queries after 2,000 positions: 26 us laid out against
-  // 28.5 staged at 12/2 heads of 128 with the key bias, but 23 against 18.8
-  // at 14/2 heads of 64, and after 32 positions 14.7 against 18.6, 12.1
-  // against 11.3 and (32/8 of 64) 12.4 against 10.5.
+  // takes, of a paged or sealing cache, where laying its pages out pays.
   // `workspace` holds chunk_workspace_bytes and belongs to the launch until
   // `done`, which its last kernel signals.
-  constexpr int kChunkQueries = 64;
   bool chunk_applies(const KVSource &kv, const AttentionArgs &a);
   std::size_t chunk_workspace_bytes(const KVSource &kv, const AttentionArgs &a);
   void launch_chunk(const KVSource &kv, const AttentionArgs &a, void *workspace, hipEvent_t done,

@@ -29,9 +29,10 @@ def mixed_map(seq):
     return [[order[(layer + i) % 4] for i in range(seq // P + 1)] for layer in range(LAYERS)]
 
 
-def chunk_case(heads, kv, hd, seq, seq_q, seed, bias, split, unread=()):
+def chunk_case(heads, kv, hd, seq, seq_q, seed, bias, split, unread=(), caches=None):
     """Stores `seq` positions, the last `seq_q` as one run, seals pages at the
-    mixed tiers, then attends the run's queries through the cache."""
+    mixed tiers, then attends the run's queries through the cache (appended to
+    `caches`)."""
     m = mi()
     d = m.device
     rng = np.random.default_rng(seed)
@@ -57,6 +58,8 @@ def chunk_case(heads, kv, hd, seq, seq_q, seed, bias, split, unread=()):
     cache.attention(1, put(q), put(b) if bias else None, rope, out, seq_q, seq, heads, kv, hd,
                     put(k[start:]), put(v[start:]), None, part)
     got = out.to_numpy().reshape(seq_q, heads, hd)
+    if caches is not None:
+        caches.append(cache)
     # The oracle: every full page's bytes and tier as the cache holds them.
     own_first = start // P
     pages, tiers = sealed_pages(alloc, 1, (seq - 1) // P)
