@@ -446,7 +446,8 @@ namespace mi
       constexpr int kStage = NP * kBlock;
       constexpr int kV = (kBias ? 2 : 1) * kP * HD; // V^T's place in a block
       constexpr int kWaveRows = RT * kTileRows;
-      extern __shared__ std::uint16_t stages[];
+      extern __shared__ u32x4 stage_words[];
+      auto *const stages = reinterpret_cast<std::uint16_t *>(stage_words);
       const int lane = threadIdx.x & 63;
       const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
       const int half = lane >> 5;
@@ -771,15 +772,13 @@ namespace mi
       args.qb = std::min(args.seq_q, block_rows(RT) / args.group);
       auto kernel = chunk_kernel<HD, RT, NP, kBias, kWavesASimd>;
       constexpr std::size_t kLds = 2 * NP * page_block<HD, kBias>() * sizeof(std::uint16_t);
-      // Workgroups the device holds at once, and the LDS limit raised, once.
+      // Workgroups the device holds at once, and the LDS limit raised, once
+      // (the stages of some shapes pass 64 KB only with the kernel's own LDS).
       static const long held = [&] {
-        if (kLds > 64 * 1024)
-        {
-          hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        static_cast<int>(kLds)),
-                    "hipFuncSetAttribute chunk LDS");
-        }
+        hip_check(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      static_cast<int>(kLds)),
+                  "hipFuncSetAttribute chunk LDS");
         int per_cu = 0;
         hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kChunkThreads, kLds),
                   "hipOccupancyMaxActiveBlocksPerMultiprocessor chunk");
