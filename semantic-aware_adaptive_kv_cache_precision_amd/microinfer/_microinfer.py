@@ -706,7 +706,7 @@ class DeviceIndex:
         return self._storage.ptr
 
 
-@functools.lru_cache(maxsize=64)
+@functools.lru_cache(maxsize=64, typed=True)
 def _attention_partials(head_dim: int) -> int:
     return int(lib.mi_attention_partials_floats(head_dim))
 
@@ -795,11 +795,11 @@ class ImportanceScores:
 
     def row(self, layer: int) -> int:
         """The device address of a layer's scores, for a fused fold."""
-        at = self._rows.get(layer)
-        if at is None:
+        at = self._rows.get(layer) if type(layer) is int else None
+        if at is None:  # (a float equal to a known layer is refused as any is)
             p = _vp()
             _check(lib.mi_scores_layer_row(self._h, layer, C.byref(p)))
-            at = self._rows[layer] = p.value
+            at = self._rows[int(layer)] = p.value
         return at
 
     def fold(self, layer: int, mass: FloatTensor, heads: int, pages: int) -> None:

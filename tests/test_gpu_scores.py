@@ -7,6 +7,8 @@ seeds its score; a refused fold changes nothing.
 GPU parity tests. Scores are compared bit for bit (importance_scores.cu:31-50,
 tests/test_importance_scores.py:85-115)."""
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -88,3 +90,17 @@ def test_a_refused_fold_changes_nothing():
         scores.fold(0, d.upload_f32(mass.ravel()), 3, 9)
     np.testing.assert_array_equal(scores.download(), before)
     assert isinstance(m.OutOfMemory("x"), MemoryError)
+
+
+def test_what_is_kept_by_a_number_is_found_by_that_number_alone():
+    """A layer's row and a head's partials, once asked for, are not also given
+    to a float that equals their number."""
+    m = mi()
+    d = m.device
+    scores = d.ImportanceScores(2, 8)
+    row, floats = scores.row(1), d.attention_partials(64)
+    for kept, number in ((scores.row, 1), (m._attention_partials, 64), (d.attention_partials, 64)):
+        kept(number)
+        with pytest.raises(ctypes.ArgumentError):
+            kept(float(number))
+    assert scores.row(1) == row and d.attention_partials(64) == floats
