@@ -483,7 +483,8 @@ namespace mi
         {
           qf[t][c] = as_half8(valid[t] ? load_global<u32x4>(q + 16 * c) : u32x4{0u, 0u, 0u, 0u});
         }
-        run[t].m = -INFINITY;
+        // (A lane with no row: every probability 0, so that it moves nothing.)
+        run[t].m = valid[t] ? -INFINITY : 1e30f;
         run[t].l = 0.0f;
 #pragma unroll
         for (int dt = 0; dt < HD / 32; ++dt)
